@@ -51,6 +51,7 @@ EXPORTS = (
     "ttcd_ttt_proj_beta_t_fwd",
     "ttcd_ttt_scan_fwd",
     "ttcd_attn_schedule_coverage",
+    "ttcd_attn_block_coverage",
 )
 
 _i32 = ctypes.c_int
@@ -133,6 +134,7 @@ _SIGS = {
         _vp, _vp, ctypes.c_float, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "ttcd_attn_schedule_coverage": (_i32, [
         _i32, _i32, _i32, _i32, _i32, _vp, _vp]),
+    "ttcd_attn_block_coverage": (_i32, [_i32, _i32, _i32, _i32, _vp, _vp]),
 }
 
 _lock = threading.Lock()

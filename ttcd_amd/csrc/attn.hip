@@ -40,9 +40,9 @@
 //     row max of S(k+1) (slot_body). In the lazy mode at D = 128 no row max
 //     is needed before the exp2, so the PV MFMAs of slot k run under the
 //     first half of S(k+1)'s exp2 instead (slot_body_lazy).
-//   * Workgroups are remapped so each XCD (own L2) sweeps a contiguous run of
-//     (b, kv head, query block, head or head pair in group); heaviest query
-//     blocks first.
+//   * Workgroups are remapped (schedule.h: BlockMap) so that the XCDs (each
+//     with its own L2) get equal shares of every (b, kv head) in runs of
+//     neighbouring query blocks, heaviest first.
 //   * Packed sequences (cu_seqlens): each workgroup builds its sequence's
 //     schedule from the sequence length, with every bound clamped to the
 //     packed tensors.
@@ -138,15 +138,6 @@ __device__ __forceinline__ float xhalf_sum(float v) {
 __device__ __forceinline__ bool xhalf_any(bool v) {
   const auto r = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
   return (r[0] | r[1]) != 0;
-}
-
-// Workgroup id -> logical id such that XCD x (which receives ids g = x, x+8,
-// ...) processes one contiguous range of logical ids.
-__device__ __forceinline__ int xcd_remap(int g, int total) {
-  constexpr int kXcd = 8;
-  const int q = total / kXcd, r = total % kXcd;
-  const int x = g % kXcd, loc = g / kXcd;
-  return x < r ? x * (q + 1) + loc : r * (q + 1) + (x - r) * q + loc;
 }
 
 template <int D>
@@ -684,17 +675,12 @@ void attn_fwd_kernel(AttnArgs a) {
   const int R = a.sched.rows;
   const int hpw = kWaveRows / R;
   const int span = kWaves * R;
-  // Workgroup -> (b, kv head, query block [heaviest first], head group),
-  // XCD-remapped: each XCD sweeps a contiguous run, so the query heads
-  // sharing a K/V head and neighbouring query blocks share its L2.
-  int rest = xcd_remap(__builtin_amdgcn_workgroup_id_x(), a.nwg);
-  const int ngrp = a.G / hpw;
-  const int g = rest % ngrp;
-  rest /= ngrp;
-  const int qb = a.qb0 + (a.nqb - 1 - rest % a.nqb);
-  rest /= a.nqb;
-  const int hk = rest % a.Hkv;
-  const int b = rest / a.Hkv;
+  // Workgroup -> (b, kv head), query block, head group (schedule.h: BlockMap).
+  int pair, qb, g;
+  if (!a.map.locate((int)__builtin_amdgcn_workgroup_id_x(), &pair, &qb, &g)) return;
+  qb += a.qb0;
+  const int b = a.hkv.quot(pair);
+  const int hk = pair - b * a.Hkv;
   const int h = hk * a.G + g * hpw;  // the wavefront's first query head
   // this lane's head is h + dh (kept out of the uniform bases below, so they
   // stay in scalar registers through the sweep)
@@ -981,18 +967,21 @@ void attn_fwd_kernel(AttnArgs a) {
 template <int D, typename T, bool DUAL>
 hipError_t launch_typed(const AttnArgs& a, hipStream_t stream) {
   AttnArgs args = a;
-  args.nwg = a.B * (a.Hq / (kWaveRows / a.sched.rows)) * a.nqb;
+  args.map = make_block_map(a.B * a.Hkv, a.nqb, a.G / (kWaveRows / a.sched.rows),
+                            a.cu_seqlens != nullptr);
+  args.hkv = make_fast_div(a.Hkv);
+  const int nwg = args.map.launched();
   // The sum-triggered lazy slot needs a second P^T buffer, which D = 64 has
   // no registers for at three waves per SIMD; D = 64 and the exact mode take
   // the max-first slot.
   if constexpr (D == 128) {
     if (a.rescale_log2 > 0.f) {
-      hipLaunchKernelGGL((attn_fwd_kernel<D, T, DUAL, true>), dim3(args.nwg), dim3(kWaves * 64),
+      hipLaunchKernelGGL((attn_fwd_kernel<D, T, DUAL, true>), dim3(nwg), dim3(kWaves * 64),
                          0, stream, args);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((attn_fwd_kernel<D, T, DUAL, false>), dim3(args.nwg), dim3(kWaves * 64), 0,
+  hipLaunchKernelGGL((attn_fwd_kernel<D, T, DUAL, false>), dim3(nwg), dim3(kWaves * 64), 0,
                      stream, args);
   return hipGetLastError();
 }

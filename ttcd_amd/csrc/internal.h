@@ -29,7 +29,8 @@ struct AttnArgs {
                   // bottom-right alignment; 0 when Tq == Tk)
   int qb0;        // first query tile launched: q_off / (4 * sched.rows)
   int nqb;        // query tiles of 4 * sched.rows tokens per (b, head group) launched
-  int nwg;        // workgroups launched (set by the launcher)
+  BlockMap map;   // workgroup ids -> query blocks (set by the launcher)
+  FastDiv hkv;    // division by Hkv (set by the launcher)
   float c;        // sm_scale * log2(e)
   float rescale_log2;  // lazy online softmax: the reference max moves when a row max
                        // exceeds it by more than 2^rescale_log2 (0: exact running max)

@@ -309,6 +309,124 @@ TTCD_HD int word_tile(uint32_t w) { return (int)(w >> kWordTileShift); }
 TTCD_HD int word_j0(const Schedule& sc, uint32_t w) { return (int)(w & ~63u) - sc.kshift; }
 TTCD_HD Band word_band(const Schedule& sc, uint32_t w) { return (w & kWordFar) ? sc.p2 : sc.p1; }
 
+// Workgroup ids -> query blocks.
+//
+// The hardware deals consecutive workgroup ids round-robin to the kXcd XCDs
+// (each with its own L2) and, inside an XCD, to its kXcdCus CUs, so id g is
+// the (g / 8)-th workgroup of XCD g % 8, and the ones 32 apart there share a
+// CU while every place is free. A call has npair = B * Hkv K/V heads, each
+// with nqb query blocks (block nqb - 1 sweeps the most keys of a causal
+// sequence) of ngrp workgroups. The blocks of a K/V head are cut into levels
+// of seg consecutive blocks, the heaviest first, and the (level, head) items
+// are dealt to the XCDs level by level: every XCD gets the same share of
+// every level of every head (of every packed sequence too), while the
+// workgroups of an item, which sweep nearly the same keys, share one L2.
+// With npair a multiple of 8 an XCD keeps whole heads; otherwise the deal
+// runs forth and back so that no XCD always gets the heavier items.
+//
+// Why: one contiguous run of (head, block) per XCD leaves the XCDs unequal
+// when a head's run is split between them (causal heads, npair not a multiple
+// of 8) or when packed sequences differ in length; the call then waits for
+// one XCD.
+//
+// Within an XCD the workgroups start heaviest first, except that the second
+// one of each CU is taken so that a CU's two add up to about the same sweep:
+// when all of them start at once nothing else evens the CUs out.
+constexpr int kXcd = 8;
+constexpr int kXcdCus = 32;
+
+// n / d for 0 <= n < 2^31 by one 64-bit product: with m = ceil(2^(31+s) / d),
+// 2^s >= d, n * m / 2^(31+s) rounds down to the quotient (Granlund and
+// Montgomery, "Division by invariant integers using multiplication", 1994).
+// A workgroup's start is a chain of scalar operations with nothing to hide
+// it, and a division by a kernel argument is ~30 of them.
+struct FastDiv {
+  uint32_t d, m;
+  int sh;
+
+  TTCD_HD int quot(int n) const { return (int)(((uint64_t)(uint32_t)n * m) >> sh); }
+};
+
+TTCD_HD FastDiv make_fast_div(int d) {
+  FastDiv f;
+  int s = 0;
+  while ((int64_t(1) << s) < d) ++s;
+  f.d = (uint32_t)d;
+  f.sh = 31 + s;
+  f.m = (uint32_t)(((uint64_t(1) << f.sh) + d - 1) / d);
+  return f;
+}
+
+struct BlockMap {
+  int nqb;               // query blocks per K/V head
+  FastDiv npair, ngrp;   // K/V heads, workgroups per block
+  FastDiv per;           // workgroups per item
+  int seg;               // blocks per item
+  int items;             // (levels) * npair
+  int rounds;            // items per XCD, rounded up
+  int snake;             // the deal changes direction every round
+
+  TTCD_HD int per_xcd() const { return rounds * (int)per.d; }
+  TTCD_HD int launched() const { return kXcd * per_xcd(); }
+
+  // Position in the heaviest-first order of an XCD's n workgroups of its
+  // i-th started one.
+  TTCD_HD int rank(int i) const {
+    const int n = per_xcd();
+    if (n <= kXcdCus) return i;
+    const int both = n < 2 * kXcdCus ? n - kXcdCus : kXcdCus;  // CUs that start with two
+    if (i >= kXcdCus) return i < kXcdCus + both ? kXcdCus + both - 1 - (i - kXcdCus) : i;
+    // the CUs that start with two take the lighter of the first kXcdCus
+    return i < both ? kXcdCus - both + i : i - both;
+  }
+
+  // The K/V head, query block and workgroup of the block that id g takes;
+  // false when it takes none.
+  TTCD_HD bool locate(int g, int* pair, int* qb, int* grp) const {
+    const int x = g % kXcd, r = rank(g / kXcd);
+    const int round = per.quot(r), in = r - round * (int)per.d;
+    const int item = round * kXcd + ((snake & round & 1) ? kXcd - 1 - x : x);
+    const int level = npair.quot(item);
+    const int blk = ngrp.quot(in);
+    *pair = item - level * (int)npair.d;
+    *grp = in - blk * (int)ngrp.d;
+    *qb = nqb - 1 - (level * seg + blk);
+    return item < items && *qb >= 0;
+  }
+};
+
+// Blocks per item. A fixed-length call whose heads are a multiple of the XCDs
+// gives each XCD whole heads. Otherwise: when every workgroup starts at once
+// on a CU of its own, as few items as give every XCD one (the sweep of the
+// heaviest workgroup is then the call, and it is fastest when the workgroups
+// beside it fetch the same tiles); when they queue, 8 items per XCD, so that
+// its share differs by little, of at least 4 blocks (whose workgroups share
+// nearly all of their tiles) and at most 32 (about what an XCD runs at once).
+//
+// Measured against one contiguous run per XCD (us, kernel time): packed
+// 12345 tokens in 9 sequences, 15/5 heads of 64, 153 -> 88; causal T = 8192,
+// 15/5 heads of 64, 230 -> 162, T = 4500 80.7 -> 67.9; 16/8 heads of 128,
+// T = 8192, 282 -> 271 and T = 4096 92.3 -> 87.2 (the order within an XCD
+// alone); 4/2 heads of 64, T = 4096, with 64 items instead of 8 50.6 -> 54.1.
+TTCD_HD BlockMap make_block_map(int npair, int nqb, int ngrp, bool packed) {
+  BlockMap m;
+  m.nqb = nqb;
+  m.npair = make_fast_div(npair);
+  m.ngrp = make_fast_div(ngrp);
+  const bool queued = (int64_t)npair * nqb * ngrp > kXcd * kXcdCus;
+  int seg = 32;
+  auto few = [&](int items) { return (int64_t)npair * ((nqb + seg - 1) / seg) < items; };
+  while (seg > 1 && few(queued && seg > 4 ? 8 * kXcd : kXcd)) seg /= 2;
+  if (!packed && npair % kXcd == 0) seg = nqb;
+  const int levels = (nqb + seg - 1) / seg;
+  m.seg = (nqb + levels - 1) / levels;
+  m.per = make_fast_div(m.seg * ngrp);
+  m.items = levels * npair;
+  m.rounds = (m.items + kXcd - 1) / kXcd;
+  m.snake = npair % kXcd != 0;
+  return m;
+}
+
 // Query rows per wavefront for a GQA group size (see Geometry): 16 rows of
 // each of two heads for an even group, else 32 rows of one head.
 #ifndef TTCD_PAIR_WAVES
