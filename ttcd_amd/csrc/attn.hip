@@ -43,6 +43,13 @@
 //   * Workgroups are remapped (schedule.h: BlockMap) so that the XCDs (each
 //     with its own L2) get equal shares of every (b, kv head) in runs of
 //     neighbouring query blocks, heaviest first.
+//   * A workgroup's start is a chain of latencies (arguments, position, plan,
+//     first tile), so the first tile and Q are requested before the plan is
+//     made, the arguments are fetched together and nothing divides; its end
+//     stores 16 bytes per lane. Together 1.6 % of 32K tokens (16/8 heads of
+//     128, windows 8192 / 4096: 1782 -> 1754 us), 5 % at windows 2048 / 1024
+//     (T = 5003, 173 -> 165 us), 8 % at 512 / 256 (T = 2048, 4/2 heads of
+//     64, 15.4 -> 14.1 us).
 //   * Packed sequences (cu_seqlens): each workgroup builds its sequence's
 //     schedule from the sequence length, with every bound clamped to the
 //     packed tensors.
@@ -85,6 +92,8 @@ namespace ttcd {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -363,15 +372,25 @@ __device__ __forceinline__ void emit(const f32x16 (&o)[Geo<D>::DT], float m, flo
   const float inv = lt > 0.f ? 1.0f / lt : 0.f;
   if (qrow >= T_ || qrow < q_off) return;  // rows of this launch only
   const int half = lane >> 5;
-  T* dst = out + (int64_t)(qrow - q_off) * o_st + half * 4;
+  // A lane holds d = 8g + 4 half .. + 3 of its row for every g. Two g's are
+  // swapped between the row's two lanes, so that each stores 8 neighbouring
+  // elements: half as many stores, of 32 contiguous bytes per row.
+  T* dst = out + (int64_t)(qrow - q_off) * o_st + half * 8;
 #pragma unroll
   for (int dt = 0; dt < Geo<D>::DT; ++dt) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      v4 w;
+    for (int g = 0; g < 4; g += 2) {
+      u32x2 w[2];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = static_cast<T>(o[dt][4 * g + e] * inv);
-      *reinterpret_cast<v4*>(dst + dt * 32 + 8 * g) = w;
+      for (int i = 0; i < 2; ++i) {
+        v4 t;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = static_cast<T>(o[dt][4 * (g + i) + e] * inv);
+        w[i] = __builtin_bit_cast(u32x2, t);
+      }
+      const auto r0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
+      const auto r1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+      *reinterpret_cast<u32x4*>(dst + dt * 32 + 8 * g) = u32x4{r0[0], r1[0], r0[1], r1[1]};
     }
   }
   if (lse != nullptr && half == 0) {
@@ -669,11 +688,16 @@ void attn_fwd_kernel(AttnArgs a) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
+  // One field of every 64-byte line of the arguments, together: read where
+  // they are used, they cost a start one cache miss after the other.
+  asm volatile("" ::"s"(a.q), "s"(a.q_sb), "s"(a.v_sb), "s"(a.B), "s"(a.sched.T),
+               "s"(a.lse_sb));
+
   // Wavefront geometry: R query rows per wavefront, 32 of one head or (hpw =
   // 2, even GQA group) 16 of each of two heads of the group; score column
   // n = lane % 32 is row n % R of head h + n / R.
   const int R = a.sched.rows;
-  const int hpw = kWaveRows / R;
+  const int hpw = R == kWaveRows ? 1 : 2;
   const int span = kWaves * R;
   // Workgroup -> (b, kv head), query block, head group (schedule.h: BlockMap).
   int pair, qb, g;
@@ -734,28 +758,13 @@ void attn_fwd_kernel(AttnArgs a) {
   x.half = lane >> 5;
   x.T_ = T_;
   x.ln = make_lane<D>(a.k_st, a.v_st, wave, lane);
-  {
-    const bool row_ok = (x.qrow < T_) & (x.qrow >= q_off);
-    const T* src = qp + (int64_t)(row_ok ? x.qrow - q_off : 0) * a.q_st + (lane >> 5) * 8;
-#pragma unroll
-    for (int ks = 0; ks < G::DK; ++ks) {
-      v8 z = {};
-      x.qf[ks] = row_ok ? *reinterpret_cast<const v8*>(src + ks * 16) : z;
-    }
-  }
-
   int n_hi = 0, n_lo = 1;
   if (!sc.wg_range(t0, t_last, &n_hi, &n_lo)) {
     n_hi = 0;
     n_lo = 1;
   }
   const int count = n_hi - n_lo + 1;
-  const SlotPlan sp = make_slot_plan(
-      sc, [&](int wv) { return t0 + wv * R; }, n_hi, n_lo);
-  // The plan is workgroup-uniform; keep it in scalar registers.
-  const int nslot = __builtin_amdgcn_readfirstlane(count > 0 ? sp.slots() : 0);
 
-  const WaveSlots wsl(sc, r0);
   const int64_t kst = a.k_st, vst = a.v_st;
   const float rescale_log2 = a.rescale_log2;
   // Byte address of tile 0's first key (key -kshift) and bytes per key: an
@@ -782,6 +791,27 @@ void attn_fwd_kernel(AttnArgs a) {
         dma_tile<D, T, false>(dst, vp, vst, word_j0(sc, w), T_, wave, lane, off, false);
     }
   };
+  // The first slot's tile is known before the plan (slot 0 is always the
+  // first pass over n_hi): its loads, and those of Q, run under the plan.
+  const uint32_t w_first =
+      count > 0 ? slot_load_word(sc, __builtin_amdgcn_readfirstlane(n_hi), T_) : 0u;
+  dma_half(true, w_first, 0);
+  dma_half(false, w_first, 0);
+  {
+    // A row outside [q_off, T) reads its nearest valid one: its column of
+    // every score is computed and never written.
+    const int row = max(min(x.qrow, T_ - 1), q_off) - q_off;
+    const T* src = qp + (int64_t)row * a.q_st + (lane >> 5) * 8;
+#pragma unroll
+    for (int ks = 0; ks < G::DK; ++ks) x.qf[ks] = *reinterpret_cast<const v8*>(src + ks * 16);
+  }
+
+  const SlotPlan sp = make_slot_plan(
+      sc, [&](int wv) { return t0 + wv * R; }, n_hi, n_lo);
+  // The plan is workgroup-uniform; keep it in scalar registers.
+  const int nslot = __builtin_amdgcn_readfirstlane(count > 0 ? sp.slots() : 0);
+
+  const WaveSlots wsl(sc, r0);
 
   f32x16 o[G::DT];
 #pragma unroll
@@ -807,12 +837,10 @@ void attn_fwd_kernel(AttnArgs a) {
     return slot_word(sc, sp, wsl, nslot, wave_valid, T_, tb + lane);
   };
   uint32_t tbl = words(0);
-  // Prologue: K(0), V(0), K(1) in LDS, scores of slot 0. w_cur and w_nxt are
-  // the words of slots 0 and 1.
+  // Prologue: K(0), V(0) (already on their way), K(1) in LDS, scores of slot
+  // 0. w_cur and w_nxt are the words of slots 0 and 1.
   uint32_t w_cur = (uint32_t)__builtin_amdgcn_readlane((int)tbl, 0);
   uint32_t w_nxt = (uint32_t)__builtin_amdgcn_readlane((int)tbl, 1);
-  dma_half(true, w_cur, 0);
-  dma_half(false, w_cur, 0);
   dma_half(true, w_nxt, 1);
   asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   // Scores of slot 0 and their lane max (unmasked; slot 0's mask and

@@ -121,7 +121,7 @@ struct SlotPlan {
   int n_hi;            // first (highest) tile
   int count;           // tiles n_hi .. n_hi - count + 1
   int ndup;            // repeated (mixed) tiles
-  int dup[kMaxDup];    // their tile indices, descending; kNoTile for unused entries
+  int dup[kMaxDup];    // their tile indices, descending, among unused entries (kNoTile)
 
   TTCD_HD int slots() const { return count + ndup; }
 
@@ -155,44 +155,27 @@ TTCD_HD int wave_mixed_tile(const Schedule& sc, int r0) {
                                                                                    : kNoTile;
 }
 
-// Slot plan of a workgroup whose wave w starts at row r0_of_wave(w) (rows >= T
-// are idle waves) and whose tiles are n_hi down to n_lo.
+// Slot plan of a workgroup whose wave w starts at row r0_of_wave(w), rising
+// with w (rows >= T are idle waves), and whose tiles are n_hi down to n_lo.
+// A later wave's mixed tile is never a lower one, and the waves without one
+// (no far key yet, or no row) are the first or the last of the workgroup: the
+// last wave's tile first, equal neighbours dropped, is the descending list.
 template <typename R0>
 TTCD_HD SlotPlan make_slot_plan(const Schedule& sc, R0 r0_of_wave, int n_hi, int n_lo) {
   SlotPlan sp;
   sp.n_hi = n_hi;
   sp.count = n_hi - n_lo + 1;
-  int* d = sp.dup;
-#pragma unroll
-  for (int w = 0; w < kMaxDup; ++w) {
-    const int r0 = r0_of_wave(w);
-    const int n = r0 < sc.T ? wave_mixed_tile(sc, r0) : kNoTile;
-    d[w] = (n >= n_lo && n <= n_hi) ? n : kNoTile;
-  }
-  // sort descending (kNoTile is the smallest int), blank out repeats, then
-  // sort again so the distinct tiles lead the array
-  auto sort_desc = [](int* v) {
-#pragma unroll
-    for (int a = 0; a < kMaxDup; ++a)
-#pragma unroll
-      for (int b = 0; b + 1 < kMaxDup - a; ++b)
-        if (v[b] < v[b + 1]) {
-          const int t = v[b];
-          v[b] = v[b + 1];
-          v[b + 1] = t;
-        }
-  };
-  sort_desc(d);
   sp.ndup = 0;
   int prev = kNoTile;
 #pragma unroll
   for (int i = 0; i < kMaxDup; ++i) {
-    const int v = d[i];
-    d[i] = (v == prev) ? kNoTile : v;
-    prev = v;
-    sp.ndup += d[i] != kNoTile;
+    const int r0 = r0_of_wave(kMaxDup - 1 - i);
+    int n = r0 < sc.T ? wave_mixed_tile(sc, r0) : kNoTile;
+    n = (n >= n_lo && n <= n_hi) ? n : kNoTile;
+    sp.dup[i] = (n == prev) ? kNoTile : n;
+    prev = n;
+    sp.ndup += sp.dup[i] != kNoTile;
   }
-  sort_desc(d);
   return sp;
 }
 
@@ -284,6 +267,13 @@ enum SlotWordBits : uint32_t {
 constexpr int kWordTileShift = 6;
 static_assert((1 << kWordTileShift) == kBlockN, "word & ~63 is the tile's key offset");
 
+// The load part of the word of a slot over tile n (keys [0, T)).
+TTCD_HD uint32_t slot_load_word(const Schedule& sc, int n, int T) {
+  const int j0 = sc.tile_start(n);
+  return (uint32_t)n << kWordTileShift | kWordLoad |
+         (((j0 >= 0) & (j0 + kBlockN <= T)) ? kWordInterior : 0u);
+}
+
 // Word of slot k of plan sp (nslot slots) for the wave described by ws
 // (wave_valid false: a wave without rows, which only loads), keys [0, T).
 TTCD_HD uint32_t slot_word(const Schedule& sc, const SlotPlan& sp, const WaveSlots& ws,
@@ -292,12 +282,9 @@ TTCD_HD uint32_t slot_word(const Schedule& sc, const SlotPlan& sp, const WaveSlo
   int n = sp.tile(k, &repeat);
   const bool load = (k >= 0) & (k < nslot);
   n = load ? n : 0;
-  const int j0 = sc.tile_start(n);
   const int act = (load & wave_valid) ? ws.act(n, repeat) : (int)kSkip;
   const bool far = (act == kBand2) | (act == kFar);
-  uint32_t w = (uint32_t)n << kWordTileShift;
-  w |= load ? kWordLoad : 0u;
-  w |= (load & (j0 >= 0) & (j0 + kBlockN <= T)) ? kWordInterior : 0u;
+  uint32_t w = load ? slot_load_word(sc, n, T) : 0u;
   w |= act != kSkip ? kWordActive : 0u;
   w |= far ? kWordFar : 0u;
   w |= act == kStudentLast ? kWordLast : 0u;
