@@ -376,6 +376,23 @@ ttcd_status ttcd_ttt_features_fwd(const void* gu_t, const void* gu_s,
                                   int inter, ttcd_dtype dtype, void* stream);
 
 /*
+ * The same pass over sequences of `tokens` positions that need not be whole
+ * chunks (nchunk = ceil(tokens / chunk)), and without what no update reads:
+ * gu_t: the teacher rows of sequence b start at row b * t_rows (tokens of
+ * them are read); gu_s: the student rows likewise at b * s_rows, only those
+ * of the first nchunk - 1 chunks. z (B * nchunk * chunk, inter) with zero
+ * rows from position `tokens` on; z_hat and diff (B * (nchunk - 1) * chunk,
+ * inter). gu_s, z_hat and diff may be NULL when nchunk == 1.
+ */
+ttcd_status ttcd_ttt_features_tokens_fwd(const void* gu_t, int64_t t_rows,
+                                         const void* gu_s, int64_t s_rows,
+                                         int64_t gu_stride, const void* conv_t,
+                                         const void* conv_s, ttcd_dtype w_dtype,
+                                         int kernel_size, void* z, void* z_hat,
+                                         void* diff, int B, int tokens, int chunk,
+                                         int inter, ttcd_dtype dtype, void* stream);
+
+/*
  * The TTT MLP's update scan around its GEMMs (the group loop of
  * custom_models/ipttcd/modeling_ipttcdv9_lowcopy_scanfuse.py:121-172).
  *

@@ -48,6 +48,7 @@ EXPORTS = (
     "ttcd_add_rmsnorm_fwd",
     "ttcd_swiglu_fwd",
     "ttcd_ttt_features_fwd",
+    "ttcd_ttt_features_tokens_fwd",
     "ttcd_ttt_proj_beta_t_fwd",
     "ttcd_ttt_scan_fwd",
     "ttcd_attn_schedule_coverage",
@@ -127,6 +128,9 @@ _SIGS = {
     "ttcd_swiglu_fwd": (_i32, [_vp, _vp, _vp, _i64, _i32, _i64, _i64, _i64, _i32, _vp]),
     "ttcd_ttt_features_fwd": (_i32, [
         _vp, _vp, _i64, _vp, _vp, _i32, _i32, _vp, _vp, _vp,
+        _i32, _i32, _i32, _i32, _i32, _vp]),
+    "ttcd_ttt_features_tokens_fwd": (_i32, [
+        _vp, _i64, _vp, _i64, _i64, _vp, _vp, _i32, _i32, _vp, _vp, _vp,
         _i32, _i32, _i32, _i32, _i32, _vp]),
     "ttcd_ttt_proj_beta_t_fwd": (_i32, [
         _vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),

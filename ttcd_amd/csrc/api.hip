@@ -810,34 +810,61 @@ ttcd_status ttcd_swiglu_fwd(const void* gate, const void* up, void* out, int64_t
                   "swiglu launch");
 }
 
-ttcd_status ttcd_ttt_features_fwd(const void* gu_t, const void* gu_s, int64_t gu_stride,
-                                  const void* conv_t, const void* conv_s, ttcd_dtype w_dtype,
-                                  int kernel_size, void* z, void* z_hat, void* diff, int B,
-                                  int nchunk, int chunk, int inter, ttcd_dtype dtype,
-                                  void* stream) {
-  if (!gu_t || !gu_s || !z || !z_hat || (nchunk > 1 && !diff))
+// Both forms of the feature pass.
+static ttcd_status ttt_features(const ttcd::TttFeatureArgs& a, ttcd_dtype w_dtype,
+                                ttcd_dtype dtype, void* stream) {
+  if (!a.gu_t || !a.z || (a.nchunk > 1 && !a.diff) ||
+      ((a.nchunk > 1 || a.last_student) && (!a.gu_s || !a.z_hat)))
     return fail(TTCD_ERR_INVALID_ARGUMENT, "null pointer argument");
-  if (B < 1 || nchunk < 1 || chunk < 1 || inter < 1)
+  if (a.B < 1 || a.nchunk < 1 || a.C < 1 || a.I < 1)
     return fail(TTCD_ERR_INVALID_ARGUMENT, "need B, nchunk, chunk, inter >= 1");
-  if (gu_stride < 2 * (int64_t)inter)
+  if (a.gu_st < 2 * (int64_t)a.I)
     return fail(TTCD_ERR_INVALID_ARGUMENT, "gate|up row stride must be >= 2 * inter");
-  if (kernel_size < 1 || ((conv_t || conv_s) && kernel_size > 8))
+  if (a.K < 1 || ((a.w_t || a.w_s) && a.K > 8))
     return fail(TTCD_ERR_UNSUPPORTED, "conv kernel size must be in 1..8");
   if (dtype != TTCD_DTYPE_BF16 && dtype != TTCD_DTYPE_F16)
     return fail(TTCD_ERR_UNSUPPORTED, "dtype must be bf16 or f16");
   if ((unsigned)w_dtype > TTCD_DTYPE_F32)
     return fail(TTCD_ERR_INVALID_ARGUMENT, "unknown conv weight dtype");
-  if (inter % 8 != 0 || gu_stride % 8 != 0)
+  if (a.I % 8 != 0 || a.gu_st % 8 != 0)
     return fail(TTCD_ERR_UNSUPPORTED, "inter and the gate|up row stride must be multiples of 8");
-  const void* all[5] = {gu_t, gu_s, z, z_hat, diff};
+  const void* all[5] = {a.gu_t, a.gu_s, a.z, a.z_hat, a.diff};
   for (int i = 0; i < 5; ++i)
     if (all[i] && !aligned16(all[i]))
       return fail(TTCD_ERR_UNSUPPORTED, "tensor base pointers must be 16-byte aligned");
-  ttcd::TttFeatureArgs a{gu_t, gu_s, gu_stride, conv_t, conv_s, (conv_t || conv_s) ? kernel_size : 1,
-                         z, z_hat, diff, B, nchunk, chunk, inter};
-  return from_hip(ttcd::launch_ttt_features(a, elem(dtype), elem(w_dtype),
+  ttcd::TttFeatureArgs k = a;
+  if (!a.w_t && !a.w_s) k.K = 1;
+  return from_hip(ttcd::launch_ttt_features(k, elem(dtype), elem(w_dtype),
                                             static_cast<hipStream_t>(stream)),
                   "ttt features launch");
+}
+
+ttcd_status ttcd_ttt_features_fwd(const void* gu_t, const void* gu_s, int64_t gu_stride,
+                                  const void* conv_t, const void* conv_s, ttcd_dtype w_dtype,
+                                  int kernel_size, void* z, void* z_hat, void* diff, int B,
+                                  int nchunk, int chunk, int inter, ttcd_dtype dtype,
+                                  void* stream) {
+  const int64_t rows = (int64_t)nchunk * chunk;
+  return ttt_features({gu_t, gu_s, gu_stride, rows, rows, conv_t, conv_s, kernel_size, z, z_hat,
+                       diff, B, nchunk, chunk, inter, rows, true},
+                      w_dtype, dtype, stream);
+}
+
+ttcd_status ttcd_ttt_features_tokens_fwd(const void* gu_t, int64_t t_rows, const void* gu_s,
+                                         int64_t s_rows, int64_t gu_stride, const void* conv_t,
+                                         const void* conv_s, ttcd_dtype w_dtype,
+                                         int kernel_size, void* z, void* z_hat, void* diff,
+                                         int B, int tokens, int chunk, int inter,
+                                         ttcd_dtype dtype, void* stream) {
+  if (tokens < 1 || chunk < 1)
+    return fail(TTCD_ERR_INVALID_ARGUMENT, "need tokens, chunk >= 1");
+  const int nchunk = (int)(((int64_t)tokens + chunk - 1) / chunk);
+  if (t_rows < tokens || (nchunk > 1 && s_rows < (int64_t)(nchunk - 1) * chunk))
+    return fail(TTCD_ERR_INVALID_ARGUMENT,
+                "t_rows must be >= tokens and s_rows >= the updating chunks' rows");
+  return ttt_features({gu_t, gu_s, gu_stride, t_rows, s_rows, conv_t, conv_s, kernel_size, z,
+                       z_hat, diff, B, nchunk, chunk, inter, tokens, false},
+                      w_dtype, dtype, stream);
 }
 
 ttcd_status ttcd_ttt_proj_beta_t_fwd(const void* pd, int64_t pd_stride, const void* beta,

@@ -83,18 +83,24 @@ hipError_t launch_dual_residual_rmsnorm(const void* a_t, const void* a_s, const 
                                         void* res_out, void* y_s, int64_t rows, int H,
                                         Elem dtype, hipStream_t stream, bool round_sum = false);
 
-// TTT MLP feature pass (ttt.hip). Rows are b-major, then chunk, then position.
+// TTT MLP feature pass (ttt.hip). z rows are b-major, then chunk, then
+// position; positions from `tokens` on are padding (z = 0). gu_t / gu_s hold
+// the positions of a sequence in consecutive rows, t_rows / s_rows from one
+// sequence to the next.
 struct TttFeatureArgs {
-  const void* gu_t;  // teacher (rows, 2*I) gate | up, row stride gu_st
+  const void* gu_t;  // teacher (.., 2*I) gate | up, row stride gu_st
   const void* gu_s;  // student, same layout
   int64_t gu_st;
+  int64_t t_rows, s_rows;
   const void* w_t;   // teacher conv weight (I, K) or null
   const void* w_s;   // student conv weight (I, K) or null
   int K;
-  void* z;           // (rows, I) teacher features
-  void* z_hat;       // (rows, I) student features after the student conv
+  void* z;           // (B * nchunk * C, I) teacher features
+  void* z_hat;       // student features after the student conv, chunks as below
   void* diff;        // (B * (nchunk - 1) * C, I)
   int B, nchunk, C, I;
+  int64_t tokens;    // positions per sequence, (nchunk - 1) * C < tokens <= nchunk * C
+  bool last_student;  // z_hat holds all nchunk chunks, else the first nchunk - 1
 };
 
 hipError_t launch_swiglu(const void* gate, const void* up, void* out, int64_t rows, int cols,

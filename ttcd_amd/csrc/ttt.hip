@@ -3,10 +3,9 @@
 // swiglu_kernel replaces fla's swiglu_fwd_kernel (fla/modules/activations.py:
 // 412-426, called by swiglu / swiglu_linear in every MLP of the model):
 //   z = (g * s) * u,  s = 1 / (1 + exp(-g)),  in fp32, rounded to the dtype.
-// swiglu reads gate / up once, with non-temporal loads; the feature pass's
-// gate / up reads stay cached, since neighbouring runs re-read their halo
-// rows. Outputs are stored normally: the next op reads them soon, from the
-// last-level cache when they fit.
+// Both passes read gate / up with non-temporal loads (each value is used
+// once, but for 4 halo rows in 64). Outputs are stored normally: the next op
+// reads them soon, from the last-level cache when they fit.
 //
 // ttt_features_kernel does, in one pass, what the TTT MLP's forward does in
 // five launches before its update GEMMs (custom_models/ipttcd/
@@ -28,11 +27,19 @@
 //
 // Layout: rows are tokens, b-major, then chunk, then position in chunk;
 // gate / up are the two halves of one (rows, 2*I) GEMM output (row stride
-// `gu_stride` elements, gate at column 0, up at column I). Each thread owns
-// 8 channels (16 bytes) of a run of kRows consecutive positions of one chunk
-// and keeps the K-1 previous rows of both feature streams in registers, as
-// the standalone conv kernel does. The halo rows at the start of a run are
-// recomputed from gate / up (L2 hits: the neighbouring run streams them).
+// `gu_stride` elements, gate at column 0, up at column I).
+//
+// The pass is bound by memory, closely followed by the vector ALU (an exp
+// and a reciprocal at quarter rate per value). A lane owns 8 channels (16
+// bytes) of a run of 8 positions, and a wavefront 8 such runs one below the
+// other: all of a lane's loads are issued before the first is used, a run's
+// K-1 halo rows come from the lanes of the run below it, and the halo of the
+// wavefront is one extra row, computed by its first K-1 runs side by side.
+// Before (one thread per run of 16, a load per row behind the arithmetic of
+// the row above, the halo recomputed by every run, expf and a division):
+// 24576 rows of 3072 channels, K = 5, 350 us = 3.5 TB/s; now 207 us = 6.0
+// TB/s, and 2048 rows of 768 channels 33 -> 15 us. Plain instead of
+// non-temporal loads 217 us; three wavefronts per SIMD (spills) 355 us.
 //
 // The update scan of the group loop (scanfuse.py:121-172) around its GEMMs:
 // ttt_pd_beta_t_kernel writes pd * beta (the projected difference scaled by
@@ -71,12 +78,23 @@ __device__ __forceinline__ T round_to(float v) {
   return static_cast<T>(v);
 }
 
+// (g * s) * u with s = 1 / (1 + exp(-g)) in fp32. exp(-g) = 2^hi (1 + lo ln 2)
+// with hi + lo = -g log2(e) to ~48 bits, and one Newton step on the
+// reciprocal: 13 VALU operations beside the two quarter-rate ones, where expf
+// and the division take 25 and more. Past |g| = 120 the exponential is 0 or
+// infinite either way; an infinite denominator keeps its reciprocal 0.
 __device__ __forceinline__ float silu_mul(float g, float u) {
-  const float s = 1.0f / (1.0f + expf(-g));
+  constexpr float kLog2e = 1.44269504088896341f;
+  constexpr float kLog2eLo = (float)(1.44269504088896340736 - (double)kLog2e);
+  constexpr float kLn2 = 0.693147180559945309f;
+  const float n = __builtin_amdgcn_fmed3f(-g, -120.f, 120.f);
+  const float hi = n * kLog2e;
+  const float lo = fmaf(n, kLog2eLo, fmaf(n, kLog2e, -hi));
+  const float d = 1.0f + __builtin_amdgcn_exp2f(hi) * fmaf(lo, kLn2, 1.0f);
+  const float r = __builtin_amdgcn_rcpf(d);
+  const float s = d < INFINITY ? fmaf(fmaf(-d, r, 1.0f), r, r) : r;
   return (g * s) * u;
 }
-
-constexpr int kRows = 16;  // positions per thread
 
 template <typename T>
 __global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ gate,
@@ -97,115 +115,208 @@ __global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ gate,
   *reinterpret_cast<u32x4*>(out + r * o_st + c) = o.raw;
 }
 
-// One fused feature row: the rounded swiglu of a (gate, up) row slice.
-template <typename T>
-__device__ __forceinline__ void swiglu_row(const T* gu, int I, float (&f)[8], V8<T>& rounded) {
-  V8<T> g, u;
-  g.raw = *reinterpret_cast<const u32x4*>(gu);
-  u.raw = *reinterpret_cast<const u32x4*>(gu + I);
+// Feature pass geometry: a wavefront owns 8 groups of 8 channels (128
+// contiguous bytes, lane % 8) of 8 consecutive runs of 8 positions (lane / 8)
+// of one chunk.
+constexpr int kRunRows = 8;
+constexpr int kSegRows = 8 * kRunRows;  // positions per wavefront
+
+// The K taps of 8 neighbouring channels (w + 8 * K elements on): 16-byte loads
+// where the weights are aligned to them.
+template <typename W, int K>
+__device__ __forceinline__ void load_taps(const W* w, bool aligned, float (&wr)[K][8]) {
+  constexpr int N = (int)(8 * K * sizeof(W) / 16);
+  union {
+    u32x4 raw[N];
+    W e[8 * K];
+  } v;
+  if (aligned) {
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    rounded.e[e] = round_to<T>(silu_mul(static_cast<float>(g.e[e]), static_cast<float>(u.e[e])));
-    f[e] = static_cast<float>(rounded.e[e]);
+    for (int i = 0; i < N; ++i) v.raw[i] = reinterpret_cast<const u32x4*>(w)[i];
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8 * K; ++i) v.e[i] = w[i];
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+#pragma unroll
+    for (int j = 0; j < K; ++j) wr[j][e] = static_cast<float>(v.e[e * K + j]);
+}
+
+template <typename T>
+__device__ __forceinline__ V8<T> swiglu8(const V8<T>& g, const V8<T>& u) {
+  V8<T> f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    f.e[e] = round_to<T>(silu_mul(static_cast<float>(g.e[e]), static_cast<float>(u.e[e])));
+  return f;
+}
+
+template <typename T>
+__device__ __forceinline__ V8<T> lane_read(const V8<T>& v, int lane) {
+  V8<T> r;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) r.raw[q] = (uint32_t)__shfl((int)v.raw[q], lane, 64);
+  return r;
+}
+
+// Chunk-local causal conv of a lane's run f, each output rounded. The K-1
+// rows before a run are the last ones of the run below it; before the first
+// run of the wavefront they are `halo`, row t held by the lanes of run t.
+template <typename T, typename W, int K>
+__device__ __forceinline__ void conv_run(const V8<T> (&f)[kRunRows], const V8<T>& halo,
+                                         const W* w, bool aligned, int lane,
+                                         V8<T> (&out)[kRunRows]) {
+  static_assert(K - 1 <= kRunRows, "the halo must lie within the previous run");
+  float wr[K][8], win[K][8];
+  load_taps<W, K>(w, aligned, wr);
+#pragma unroll
+  for (int t = 0; t < K - 1; ++t) {
+    const V8<T> a = lane_read(f[kRunRows - (K - 1) + t], lane - 8);
+    const V8<T> h = lane_read(halo, 8 * t + (lane & 7));
+#pragma unroll
+    for (int e = 0; e < 8; ++e) win[t][e] = static_cast<float>(lane < 8 ? h.e[e] : a.e[e]);
+  }
+#pragma unroll
+  for (int r = 0; r < kRunRows; ++r) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      win[K - 1][e] = static_cast<float>(f[r].e[e]);
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < K; ++j) acc = fmaf(win[j][e], wr[j][e], acc);
+      out[r].e[e] = round_to<T>(acc);
+    }
+#pragma unroll
+    for (int t = 0; t < K - 1; ++t)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) win[t][e] = win[t + 1][e];
   }
 }
 
 // CT / CS: the teacher / student conv is present (else identity).
 template <typename T, typename W, int K, bool CT, bool CS>
-__global__ __launch_bounds__(256) void ttt_features_kernel(
-    const T* __restrict__ gu_t, const T* __restrict__ gu_s, int64_t gu_st,
-    const W* __restrict__ w_t, const W* __restrict__ w_s, T* __restrict__ z,
-    T* __restrict__ z_hat, T* __restrict__ diff, int B, int nchunk, int C, int I, int nseg) {
-  const int ng = I / 8;
-  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t total = (int64_t)B * nchunk * nseg * ng;
-  if (gid >= total) return;
-  const int dg = (int)(gid % ng);
-  int64_t rest = gid / ng;
-  const int seg = (int)(rest % nseg);
+__global__ __launch_bounds__(256, 2) void ttt_features_kernel(TttFeatureArgs a, int nseg,
+                                                              int ntile, int64_t waves,
+                                                              bool w_aligned) {
+  const int lane = threadIdx.x & 63;
+  const int64_t wid = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+  if (wid >= waves) return;  // whole wavefronts leave
+  const int tile = (int)(wid % ntile);
+  int rest = (int)(wid / ntile);
+  const int seg = rest % nseg;
   rest /= nseg;
-  const int ch = (int)(rest % nchunk);
-  const int b = (int)(rest / nchunk);
-  const int d0 = dg * 8;
-  const int c0 = seg * kRows;
-  const int64_t row0 = ((int64_t)b * nchunk + ch) * C;  // first token row of the chunk
-  const bool has_diff = ch < nchunk - 1;
-  const int64_t drow0 = ((int64_t)b * (nchunk - 1) + ch) * C;
+  const int ch = rest % a.nchunk;
+  const int b = rest / a.nchunk;
+  const int ng = a.I / 8, dg = tile * 8 + (lane & 7);
+  const bool col_ok = dg < ng;
+  const int d0 = (col_ok ? dg : ng - 1) * 8;  // idle lanes read a valid group, store nothing
+  const int cb = seg * kSegRows;              // first position of the wavefront in its chunk
+  const int c0 = cb + (lane >> 3) * kRunRows;
+  const int rows = col_ok ? max(0, min(kRunRows, a.C - c0)) : 0;
+  const int64_t chunk0 = (int64_t)ch * a.C;
+  const int64_t p0 = chunk0 + c0;  // first position of the run in its sequence
+  const bool has_diff = ch < a.nchunk - 1;
+  const bool has_s = has_diff || a.last_student;
 
-  float wt[K][8], ws[K][8];
+  const T* gt = static_cast<const T*>(a.gu_t) + (int64_t)b * a.t_rows * a.gu_st + d0;
+  const T* gs = static_cast<const T*>(a.gu_s) + (int64_t)b * a.s_rows * a.gu_st + d0;
+  // Positions past the chunk or the sequence read the last one before (those
+  // past the sequence are written as zero, the others not at all).
+  const int64_t last = min(a.tokens, chunk0 + a.C) - 1;
+  auto at = [&](int64_t p) { return min(p, last) * a.gu_st; };
+  // halo row t (chunk position cb - (K-1) + t) by the lanes of run t
+  const bool history = K > 1 && cb > 0;
+  const int64_t ph = chunk0 + (history ? cb - (K - 1) + min(lane >> 3, K - 2) : 0);
+
+  // every load of the teacher, then of the student, before the first is used
+  V8<T> g[kRunRows], u[kRunRows], gh, uh, g2[kRunRows], u2[kRunRows], gh2, uh2;
+  auto load = [](const T* p) {
+    V8<T> v;
+    v.raw = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+    return v;
+  };
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
+  for (int r = 0; r < kRunRows; ++r) {
+    g[r] = load(gt + at(p0 + r));
+    u[r] = load(gt + at(p0 + r) + a.I);
+  }
+  if (has_diff && CT && history) {
+    gh = load(gt + at(ph));
+    uh = load(gt + at(ph) + a.I);
+  }
+  if (has_s) {
 #pragma unroll
-    for (int j = 0; j < K; ++j) {
-      wt[j][e] = CT ? static_cast<float>(w_t[(int64_t)(d0 + e) * K + j]) : 0.f;
-      ws[j][e] = CS ? static_cast<float>(w_s[(int64_t)(d0 + e) * K + j]) : 0.f;
+    for (int r = 0; r < kRunRows; ++r) {
+      g2[r] = load(gs + at(p0 + r));
+      u2[r] = load(gs + at(p0 + r) + a.I);
     }
-
-  // wt_win / ws_win[t]: rounded features of position c - (K-1) + t
-  float twin[K][8], swin[K][8];
-#pragma unroll
-  for (int t = 0; t < K - 1; ++t) {
-    const int c = c0 - (K - 1) + t;
-    if (c >= 0) {
-      V8<T> dummy;
-      swiglu_row(gu_t + (row0 + c) * gu_st + d0, I, twin[t], dummy);
-      swiglu_row(gu_s + (row0 + c) * gu_st + d0, I, swin[t], dummy);
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) twin[t][e] = swin[t][e] = 0.f;
+    if (CS && history) {
+      gh2 = load(gs + at(ph));
+      uh2 = load(gs + at(ph) + a.I);
     }
   }
 
-  const int rows = min(kRows, C - c0);
-  for (int r = 0; r < rows; ++r) {
-    const int64_t row = row0 + c0 + r;
-    V8<T> zt, zs;
-    swiglu_row(gu_t + row * gu_st + d0, I, twin[K - 1], zt);
-    swiglu_row(gu_s + row * gu_st + d0, I, swin[K - 1], zs);
-    *reinterpret_cast<u32x4*>(z + row * I + d0) = zt.raw;
-    V8<T> tg, sh, df;
+  V8<T> f[kRunRows], tgt[kRunRows];
+  T* z = static_cast<T*>(a.z) + (((int64_t)b * a.nchunk + ch) * a.C + c0) * a.I + d0;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float at = 0.f, as = 0.f;
-      if (CT) {
+  for (int r = 0; r < kRunRows; ++r) {
+    f[r] = swiglu8(g[r], u[r]);
+    if (p0 + r >= a.tokens) f[r].raw = u32x4{0u, 0u, 0u, 0u};
+    if (r < rows) *reinterpret_cast<u32x4*>(z + (int64_t)r * a.I) = f[r].raw;
+  }
+  if (!has_s) return;
+  V8<T> halo;
+  if (has_diff) {
+    if constexpr (CT) {
+      halo.raw = u32x4{0u, 0u, 0u, 0u};
+      if (history) halo = swiglu8(gh, uh);
+      conv_run<T, W, K>(f, halo, static_cast<const W*>(a.w_t) + (int64_t)d0 * K, w_aligned, lane,
+                        tgt);
+    } else {
 #pragma unroll
-        for (int j = 0; j < K; ++j) at = fmaf(twin[j][e], wt[j][e], at);
-        tg.e[e] = round_to<T>(at);
-      } else {
-        tg.e[e] = zt.e[e];
-      }
-      if (CS) {
-#pragma unroll
-        for (int j = 0; j < K; ++j) as = fmaf(swin[j][e], ws[j][e], as);
-        sh.e[e] = round_to<T>(as);
-      } else {
-        sh.e[e] = zs.e[e];
-      }
-      df.e[e] = round_to<T>(static_cast<float>(tg.e[e]) - static_cast<float>(sh.e[e]));
+      for (int r = 0; r < kRunRows; ++r) tgt[r] = f[r];
     }
-    *reinterpret_cast<u32x4*>(z_hat + row * I + d0) = sh.raw;
-    if (has_diff)
-      *reinterpret_cast<u32x4*>(diff + (drow0 + c0 + r) * I + d0) = df.raw;
+  }
 #pragma unroll
-    for (int t = 0; t < K - 1; ++t)
+  for (int r = 0; r < kRunRows; ++r) f[r] = swiglu8(g2[r], u2[r]);
+  V8<T> sh[kRunRows];
+  if constexpr (CS) {
+    halo.raw = u32x4{0u, 0u, 0u, 0u};
+    if (history) halo = swiglu8(gh2, uh2);
+    conv_run<T, W, K>(f, halo, static_cast<const W*>(a.w_s) + (int64_t)d0 * K, w_aligned, lane,
+                      sh);
+  } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        twin[t][e] = twin[t + 1][e];
-        swin[t][e] = swin[t + 1][e];
-      }
+    for (int r = 0; r < kRunRows; ++r) sh[r] = f[r];
+  }
+  const int64_t up_row = ((int64_t)b * (a.nchunk - 1) + ch) * a.C + c0;
+  T* zh = static_cast<T*>(a.z_hat) + d0 +
+          (a.last_student ? ((int64_t)b * a.nchunk + ch) * a.C + c0 : up_row) * a.I;
+  T* df = static_cast<T*>(a.diff) + up_row * a.I + d0;
+#pragma unroll
+  for (int r = 0; r < kRunRows; ++r) {
+    if (r < rows) *reinterpret_cast<u32x4*>(zh + (int64_t)r * a.I) = sh[r].raw;
+    if (has_diff) {
+      V8<T> d;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        d.e[e] = round_to<T>(static_cast<float>(tgt[r].e[e]) - static_cast<float>(sh[r].e[e]));
+      if (r < rows) *reinterpret_cast<u32x4*>(df + (int64_t)r * a.I) = d.raw;
+    }
   }
 }
 
 template <typename T, typename W, int K, bool CT, bool CS>
 hipError_t launch_feat(const TttFeatureArgs& a, hipStream_t st) {
-  const int nseg = (a.C + kRows - 1) / kRows;
-  const int64_t total = (int64_t)a.B * a.nchunk * nseg * (a.I / 8);
-  const int64_t blocks = (total + 255) / 256;
+  const int nseg = (a.C + kSegRows - 1) / kSegRows;
+  const int ntile = (a.I / 8 + 7) / 8;
+  const int64_t waves = (int64_t)a.B * a.nchunk * nseg * ntile;
+  const int64_t blocks = (waves + 3) / 4;
+  const bool w_aligned = reinterpret_cast<uintptr_t>(a.w_t) % 16 == 0 &&
+                         reinterpret_cast<uintptr_t>(a.w_s) % 16 == 0;
   hipLaunchKernelGGL((ttt_features_kernel<T, W, K, CT, CS>), dim3((unsigned)blocks), dim3(256), 0,
-                     st, static_cast<const T*>(a.gu_t), static_cast<const T*>(a.gu_s), a.gu_st,
-                     static_cast<const W*>(a.w_t), static_cast<const W*>(a.w_s),
-                     static_cast<T*>(a.z), static_cast<T*>(a.z_hat), static_cast<T*>(a.diff), a.B,
-                     a.nchunk, a.C, a.I, nseg);
+                     st, a, nseg, ntile, waves, w_aligned);
   return hipGetLastError();
 }
 
