@@ -46,3 +46,23 @@ def test_features_at_tile_edges(gpu, B, nchunk, C, I, K, dtype, wdt, shift):
     assert torch.equal(zh.cpu(), want_zh.reshape(-1, I))
     want = (tgt[:, :-1].float() - want_zh[:, :-1].float()).to(dtype).reshape(-1, I)
     assert torch.equal(diff.cpu(), want)
+
+
+@pytest.mark.parametrize("B,tokens,C,I,ct,cs", [
+    (1, 100, 64, 64, True, True), (2, 129, 64, 72, True, False), (3, 65, 32, 64, False, True),
+    (2, 128, 64, 64, True, True), (1, 4097, 4096, 64, True, True), (2, 50, 7, 8, False, False)])
+@torch.inference_mode()
+def test_features_of_tokens_equal_the_padded_pass(gpu, B, tokens, C, I, ct, cs):
+    """Sequences that are not whole chunks: the features of the zero-padded rows,
+    bit for bit, from unpadded rows with nothing after the last one needed."""
+    nchunk, K = -(-tokens // C), 5
+    upd = (nchunk - 1) * C
+    (gu_t, gu_s), (w_t, w_s) = _inputs(B * tokens, I, K, torch.bfloat16, torch.bfloat16,
+                                       tokens + I, 0)
+    w_t, w_s = w_t if ct else None, w_s if cs else None
+    z, zh, diff = ttt._features_tokens(gu_t, gu_s[:(B - 1) * tokens + upd], w_t, w_s, B, tokens, C)
+    pad = [torch.nn.functional.pad(v.view(B, tokens, 2 * I), (0, 0, 0, nchunk * C - tokens))
+           .reshape(-1, 2 * I) for v in (gu_t, gu_s)]
+    wz, wzh, wdiff = ttt.ttt_features(pad[0], pad[1], w_t, w_s, B, nchunk, C)
+    assert torch.equal(z, wz.view(B, nchunk * C, I)) and torch.equal(diff, wdiff)
+    assert torch.equal(zh, wzh.view(B, nchunk * C, I)[:, :upd].reshape(-1, I))

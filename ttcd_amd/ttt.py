@@ -87,19 +87,8 @@ def swiglu_mlp(x: torch.Tensor, gate_up_w: torch.Tensor, down_w: torch.Tensor) -
     return F.linear(z, down_w)
 
 
-def ttt_features(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tensor | None,
-                 conv_s: torch.Tensor | None, B: int, nchunk: int, chunk: int):
-    """gu_t / gu_s: (B*nchunk*chunk, 2*I) gate|up rows of the teacher / student.
-    conv_*: (I, K) (or the module's (I, 1, K)) depthwise causal conv weights or
-    None. Returns (z, z_hat, diff): z (rows, I) teacher features, z_hat the
-    student's after its conv, diff = conv_t(z) - z_hat for every chunk but the
-    last of each batch row, (B*(nchunk-1)*chunk, I)."""
-    rows = B * nchunk * chunk
-    if gu_t.shape != gu_s.shape or gu_t.dim() != 2 or gu_t.shape[0] != rows:
-        raise ValueError(f"ttt_features: gate|up must be ({rows}, 2*I), got {tuple(gu_t.shape)}")
-    if gu_t.stride() != gu_s.stride() or gu_t.stride(1) != 1:
-        raise ValueError("ttt_features: teacher and student gate|up must share a row stride")
-    I = gu_t.shape[1] // 2
+def _conv_weights(conv_t: torch.Tensor | None, conv_s: torch.Tensor | None, I: int):
+    """([conv_t, conv_s] as contiguous (I, K) or None, their dtype, K)."""
     # Every present weight must have the first present weight's kernel size:
     # the kernel reads K taps of each, so a shorter one would be over-read.
     ws = []
@@ -114,14 +103,27 @@ def ttt_features(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tensor | 
         if K is not None and w2.shape[1] != K:
             raise ValueError("ttt_features: both convs must share a kernel size")
         K = w2.shape[1]
-        ws.append(w2)
-    if K is None:
-        K = 1
+        ws.append(w2.contiguous())
     if ws[0] is not None and ws[1] is not None and ws[0].dtype != ws[1].dtype:
         raise ValueError("ttt_features: both conv weights must share a dtype")
+    return ws, next((w.dtype for w in ws if w is not None), torch.float32), K or 1
+
+
+def ttt_features(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tensor | None,
+                 conv_s: torch.Tensor | None, B: int, nchunk: int, chunk: int):
+    """gu_t / gu_s: (B*nchunk*chunk, 2*I) gate|up rows of the teacher / student.
+    conv_*: (I, K) (or the module's (I, 1, K)) depthwise causal conv weights or
+    None. Returns (z, z_hat, diff): z (rows, I) teacher features, z_hat the
+    student's after its conv, diff = conv_t(z) - z_hat for every chunk but the
+    last of each batch row, (B*(nchunk-1)*chunk, I)."""
+    rows = B * nchunk * chunk
+    if gu_t.shape != gu_s.shape or gu_t.dim() != 2 or gu_t.shape[0] != rows:
+        raise ValueError(f"ttt_features: gate|up must be ({rows}, 2*I), got {tuple(gu_t.shape)}")
+    if gu_t.stride() != gu_s.stride() or gu_t.stride(1) != 1:
+        raise ValueError("ttt_features: teacher and student gate|up must share a row stride")
+    I = gu_t.shape[1] // 2
+    ws, wdt, K = _conv_weights(conv_t, conv_s, I)
     _check_gpu("ttt_features", gu_t=gu_t, gu_s=gu_s, conv_t=conv_t, conv_s=conv_s)
-    ws = [w.contiguous() if w is not None else None for w in ws]
-    wdt = next((w.dtype for w in ws if w is not None), torch.float32)
     dev, dt = gu_t.device, gu_t.dtype
     z = torch.empty(rows, I, dtype=dt, device=dev)
     z_hat = torch.empty(rows, I, dtype=dt, device=dev)
@@ -135,16 +137,46 @@ def ttt_features(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tensor | 
     return z, z_hat, diff
 
 
-def _stack_rows(x: torch.Tensor, t: torch.Tensor) -> torch.Tensor:
-    """(2*rows, H) view of [x; t] when they are adjacent halves of one buffer,
-    else a copy."""
+def _features_tokens(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tensor | None,
+                     conv_s: torch.Tensor | None, B: int, tokens: int, chunk: int):
+    """ttt_features for sequences of `tokens` positions of which the last chunk may
+    be part: gu_t (B * tokens, 2*I); gu_s the student's rows of the same
+    sequences, tokens apart, at least to the end of the last sequence's last
+    full update chunk. Returns z (B, nchunk*chunk, I), zero past the tokens,
+    and z_hat and diff of the first nchunk - 1 chunks, (B*(nchunk-1)*chunk, I)."""
+    I = gu_t.shape[1] // 2
+    nchunk = -(-tokens // chunk)
+    upd = (nchunk - 1) * chunk
+    if (gu_t.dim() != 2 or gu_s.dim() != 2 or gu_t.shape[0] != B * tokens
+            or gu_s.shape[0] < (B - 1) * tokens + upd or gu_s.shape[1] != gu_t.shape[1]
+            or gu_s.dtype != gu_t.dtype or gu_t.stride() != gu_s.stride()
+            or gu_t.stride(1) != 1):
+        raise ValueError("ttt_features: gate|up rows do not match the sequences")
+    ws, wdt, K = _conv_weights(conv_t, conv_s, I)
+    _check_gpu("ttt_features", gu_t=gu_t, gu_s=gu_s, conv_t=conv_t, conv_s=conv_s)
+    dev, dt = gu_t.device, gu_t.dtype
+    z = torch.empty(B, nchunk * chunk, I, dtype=dt, device=dev)
+    z_hat = torch.empty(B * upd, I, dtype=dt, device=dev)
+    diff = torch.empty(B * upd, I, dtype=dt, device=dev)
+    _lib.check(_lib.lib().ttcd_ttt_features_tokens_fwd(
+        gu_t.data_ptr(), tokens, gu_s.data_ptr(), tokens, gu_t.stride(0),
+        ws[0].data_ptr() if ws[0] is not None else None,
+        ws[1].data_ptr() if ws[1] is not None else None, _DT[wdt], K, z.data_ptr(),
+        z_hat.data_ptr(), diff.data_ptr(), B, tokens, chunk, I, _DT[dt], _stream(gu_t)))
+    return z, z_hat, diff
+
+
+def _gate_up(x: torch.Tensor, t: torch.Tensor, gate_up: torch.Tensor, n: int):
+    """gate|up of all of x's rows and of t's first n: one GEMM when x and t are
+    adjacent halves of one buffer, else two (no copy of either)."""
     H = x.shape[-1]
-    n = x.numel()
-    if (x.is_contiguous() and t.is_contiguous()
-            and t.data_ptr() == x.data_ptr() + n * x.element_size()
+    x, t = x.contiguous(), t.contiguous()
+    rows = x.numel() // H
+    if (t.data_ptr() == x.data_ptr() + x.numel() * x.element_size()
             and x.untyped_storage().data_ptr() == t.untyped_storage().data_ptr()):
-        return torch.as_strided(x, (2 * (n // H), H), (H, 1))
-    return torch.cat([x.reshape(-1, H), t.reshape(-1, H)], dim=0)
+        gu = F.linear(torch.as_strided(x, (rows + n, H), (H, 1)), gate_up)
+        return gu[:rows], gu[rows:]
+    return F.linear(x.view(rows, H), gate_up), F.linear(t.view(rows, H)[:n], gate_up)
 
 
 def proj_beta_t(pd: torch.Tensor, beta: torch.Tensor | None, B: int, nupd: int,
@@ -273,78 +305,87 @@ def ttt_mlp(x: torch.Tensor, t: torch.Tensor, w: TttMlpWeights, *, chunk: int, l
     C = chunk
     I = w.gate_up.shape[0] // 2
     nchunk = (L + C - 1) // C
-    pad = nchunk * C - L
     dt, dev = x.dtype, x.device
-    if pad:
-        x = F.pad(x, (0, 0, 0, pad))
-        t = F.pad(t, (0, 0, 0, pad))
-    rows = B * nchunk * C
-    gu = F.linear(_stack_rows(x, t), w.gate_up)  # one GEMM over teacher and student rows
-    gu_t, gu_s = gu[:rows], gu[rows:]
     if conv not in ("kernel", "stock"):
         raise ValueError(f"ttt_mlp: conv must be 'kernel' or 'stock', got {conv!r}")
     if scan not in ("kernel", "torch"):
         raise ValueError(f"ttt_mlp: scan must be 'kernel' or 'torch', got {scan!r}")
+    if L < 1 or t.numel() != x.numel() or t.dtype != dt or t.device != dev:
+        raise ValueError(f"ttt_mlp: need two matching non-empty (B, L, H) inputs, got "
+                         f"{tuple(x.shape)} {dt}, {tuple(t.shape)} {t.dtype}")
+    t = t.reshape(B, L, H).contiguous()
+    if nchunk == 1:
+        # no update: the plain MLP on the teacher's rows
+        if fused and conv == "kernel" and _conv_weights(w.conv_t, w.conv_s, I)[2] > 8:
+            raise _lib.TTCDError(_lib.TTCD_ERR_UNSUPPORTED, "conv kernel size must be in 1..8")
+        return swiglu_mlp(x, w.gate_up, w.down)
+    # The student's features are read by the updates, so never those of the
+    # last chunk: its gate|up rows stop at the end of the last full one.
+    upd = (nchunk - 1) * C
+    gu_t, gu_s = _gate_up(x, t, w.gate_up, (B - 1) * L + upd)
     if fused and conv == "kernel":
-        z, z_hat, diff = ttt_features(gu_t, gu_s, w.conv_t, w.conv_s, B, nchunk, C)
+        z, z_hat, diff = _features_tokens(gu_t, gu_s, w.conv_t, w.conv_s, B, L, C)
     else:
-        z = swiglu(gu_t[:, :I], gu_t[:, I:])
-        z_raw = swiglu(gu_s[:, :I], gu_s[:, I:])
+        z = torch.empty(B, nchunk * C, I, dtype=dt, device=dev)
+        z_raw = torch.empty(B, upd, I, dtype=dt, device=dev)
+        z[:, L:].zero_()
+        for b in range(B):
+            rt, rs = gu_t[b * L:(b + 1) * L], gu_s[b * L:b * L + upd]
+            swiglu(rt[:, :I], rt[:, I:], out=z[b, :L])
+            swiglu(rs[:, :I], rs[:, I:], out=z_raw[b])
 
         def apply_conv(v, cw):
             if cw is None:
                 return v
             if conv == "stock":
-                return stock_conv(v.view(B, nchunk, C, I), cw).view(rows, I)
-            return causal_dwconv_x(v.view(B * nchunk, C, I), cw.reshape(I, -1)).view(rows, I)
+                return stock_conv(v, cw)
+            return causal_dwconv_x(v, cw.reshape(I, -1))
 
-        z_tgt = apply_conv(z, w.conv_t)
-        z_hat = apply_conv(z_raw, w.conv_s)
-        keep = torch.arange(nchunk, device=dev) < nchunk - 1
-        diff = (z_tgt.view(B, nchunk, C, I)[:, keep] - z_hat.view(B, nchunk, C, I)[:, keep])
-        diff = diff.reshape(-1, I)
+        z_tgt = apply_conv(z.view(B, nchunk, C, I), w.conv_t)
+        z_hat = apply_conv(z_raw.view(B, nchunk - 1, C, I), w.conv_s)
+        diff = (z_tgt[:, :nchunk - 1] - z_hat).reshape(-1, I)
 
     W_base = w.down                                   # (H, I)
     z4 = z.view(B, nchunk, C, I)
+    zh4 = z_hat.view(B, nchunk - 1, C, I)
     out = torch.empty(B, nchunk, C, H, dtype=dt, device=dev)
-    if nchunk > 1:
-        beta = None
-        if w.b_proj is not None:
-            # (t_padded @ b_proj).sigmoid(), bf16 (scanfuse.py:72-74)
-            beta = torch.matmul(t.view(B, nchunk, C, H), w.b_proj).sigmoid()
-        W_upd_t = W_base.t()
-        if w.ttt_proj is not None:
-            W_upd_t = torch.matmul(W_base.t(), w.ttt_proj)  # (I, H), scanfuse.py:95-96
-        pd = torch.mm(diff, W_upd_t)                  # (B*(nchunk-1)*C, H)
-        if scan == "kernel":
-            _scan_kernel(pd, beta, z4, z_hat.view(B, nchunk, C, I), W_base, out, lr=lr,
-                         update_every=update_every)
-            return out.view(B, nchunk * C, H)[:, :L]
-        pd = pd.view(B, nchunk - 1, C, H)
-        if beta is not None:
-            pd = pd * beta[:, :nchunk - 1, :, None]
-        zh4 = z_hat.view(B, nchunk, C, I)
-        dW = torch.empty(B, nchunk - 1, H, I, dtype=dt, device=dev)
-        for b in range(B):
-            for c in range(nchunk - 1):
-                torch.mm(pd[b, c].t(), zh4[b, c], out=dW[b, c])
-        lr_t = torch.tensor(lr, dtype=dt, device=dev)
-        G = max(1, min(nchunk, update_every))
-        for b in range(B):
-            W_cur = W_base
-            for gs in range(0, nchunk, G):
-                ge = min(gs + G, nchunk)
-                upd_end = min(ge, nchunk - 1)
-                cs = lr_t * torch.cumsum(dW[b, gs:upd_end], dim=0) if upd_end > gs else None
-                for ci in range(gs, ge):
-                    if ci == gs or cs is None:
-                        W_step = W_cur
-                    else:
-                        W_step = W_cur + cs[min(ci - gs - 1, upd_end - gs - 1)]
-                    torch.mm(z4[b, ci], W_step.t(), out=out[b, ci])
-                if cs is not None:
-                    W_cur = W_cur + cs[-1]
-    else:
-        for b in range(B):
-            torch.mm(z4[b, 0], W_base.t(), out=out[b, 0])
+    beta = None
+    if w.b_proj is not None:
+        # (t_padded @ b_proj).sigmoid(), bf16 (scanfuse.py:72-74)
+        # for the updating chunks (of a batch: for all rows, then cut). Rows as
+        # a matrix: with a leading dimension torch takes a GEMM of one column,
+        # 33 us instead of 15 for 20480 rows of 1024.
+        rows = t.view(B * L, H) if B > 1 else t[0, :upd]
+        beta = torch.matmul(rows, w.b_proj).sigmoid()
+        beta = beta.view(B, -1)[:, :upd].reshape(B, nchunk - 1, C).contiguous()
+    W_upd_t = W_base.t()
+    if w.ttt_proj is not None:
+        W_upd_t = torch.matmul(W_base.t(), w.ttt_proj)  # (I, H), scanfuse.py:95-96
+    pd = torch.mm(diff, W_upd_t)                  # (B*(nchunk-1)*C, H)
+    if scan == "kernel":
+        _scan_kernel(pd, beta, z4, zh4, W_base, out, lr=lr, update_every=update_every)
+        return out.view(B, nchunk * C, H)[:, :L]
+    pd = pd.view(B, nchunk - 1, C, H)
+    if beta is not None:
+        pd = pd * beta[..., None]
+    dW = torch.empty(B, nchunk - 1, H, I, dtype=dt, device=dev)
+    for b in range(B):
+        for c in range(nchunk - 1):
+            torch.mm(pd[b, c].t(), zh4[b, c], out=dW[b, c])
+    lr_t = torch.tensor(lr, dtype=dt, device=dev)
+    G = max(1, min(nchunk, update_every))
+    for b in range(B):
+        W_cur = W_base
+        for gs in range(0, nchunk, G):
+            ge = min(gs + G, nchunk)
+            upd_end = min(ge, nchunk - 1)
+            cs = lr_t * torch.cumsum(dW[b, gs:upd_end], dim=0) if upd_end > gs else None
+            for ci in range(gs, ge):
+                if ci == gs or cs is None:
+                    W_step = W_cur
+                else:
+                    W_step = W_cur + cs[min(ci - gs - 1, upd_end - gs - 1)]
+                torch.mm(z4[b, ci], W_step.t(), out=out[b, ci])
+            if cs is not None:
+                W_cur = W_cur + cs[-1]
     return out.view(B, nchunk * C, H)[:, :L]
