@@ -128,6 +128,40 @@ ttcd_status ttcd_band_attn_kv_fwd(
     float rescale_log2, ttcd_dtype dtype, void* stream);
 
 /*
+ * The same two calls with a workspace (device memory, 16-byte aligned), with
+ * which a cached prefill of few query rows over many keys may be split over
+ * the keys: the band is cut into parts that different workgroups sweep, and
+ * their fp32 partials are added through their LSEs. Results then agree with
+ * the calls above to rounding instead of bit for bit.
+ * ttcd_attn_kv_workspace_bytes gives the bytes the split of a call needs, 0
+ * when it would not be split (Tq == Tk, rescale_log2 == 0, a short band, or
+ * enough query rows to fill the GPU); with fewer bytes, or a null or
+ * misaligned workspace, the call is not split. band_lo, band_mid, band_hi: 0,
+ * window_s, window_t of a dual call; band_lo, band_hi, band_hi of a band call
+ * (band_hi < 0: Tk). The workspace is not read before it is written; calls
+ * that may overlap in time need one each.
+ */
+size_t ttcd_attn_kv_workspace_bytes(int B, int Tq, int Tk, int Hq, int Hkv,
+                                    int D, int band_lo, int band_mid,
+                                    int band_hi, float rescale_log2);
+
+ttcd_status ttcd_dual_window_attn_kv_ws_fwd(
+    const void* q, const void* k, const void* v, void* o_t, void* o_s,
+    float* lse_t, float* lse_s, int B, int Tq, int Tk, int Hq, int Hkv, int D,
+    const int64_t q_stride[4], const int64_t k_stride[4],
+    const int64_t v_stride[4], const int64_t o_stride[4], int window_t,
+    int window_s, float sm_scale, float rescale_log2, ttcd_dtype dtype,
+    void* workspace, size_t workspace_bytes, void* stream);
+
+ttcd_status ttcd_band_attn_kv_ws_fwd(
+    const void* q, const void* k, const void* v, void* o, float* lse, int B,
+    int Tq, int Tk, int Hq, int Hkv, int D, const int64_t q_stride[4],
+    const int64_t k_stride[4], const int64_t v_stride[4],
+    const int64_t o_stride[4], int band_lo, int band_hi, float sm_scale,
+    float rescale_log2, ttcd_dtype dtype, void* workspace,
+    size_t workspace_bytes, void* stream);
+
+/*
  * Packed variable-length sequences (flash-attention's varlen layout): the
  * same two calls on nseq sequences packed along the token axis. Sequence b
  * is rows cu_seqlens[b] .. cu_seqlens[b+1]-1 of q, k, v and the outputs;

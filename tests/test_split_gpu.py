@@ -1,0 +1,114 @@
+"""Cached prefills split over keys (ttcd_attn_kv_workspace_bytes > 0).
+
+The parts fold the same scores in the same tiles as the whole call, each
+against its own reference max, and are added in fp32; so a split call is held
+to the whole call (the C entry without a workspace, itself held to the oracle
+by test_kv_attn_gpu.py) by the rounding of the probabilities and of the
+result: each probability is rounded to the input dtype in both calls, against
+different references, so a row's output may move by 2 u sum_j p_j |v_j| (u the
+dtype's unit roundoff) plus one unit of the result's own rounding, and its LSE
+only by fp32 sums (of up to 8192 terms, 1e-5)."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from conftest import make_qkv
+from ttcd_amd import _lib, fused_dual_window_attn, window_attn
+
+DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}
+
+
+def _bytes(B, Tq, Tk, H, HK, D, lo, mid, hi, rescale=8.0):
+    return _lib.lib().ttcd_attn_kv_workspace_bytes(B, Tq, Tk, H, HK, D, lo, mid, hi, rescale)
+
+
+def test_what_is_split():
+    one = 300 * 16 * 129 * 4  # bytes of one part
+    n = _bytes(1, 300, 8491, 16, 8, 128, 0, 8192, 8192)
+    assert n % one == 0 and 2 <= n // one <= 32
+    assert _bytes(1, 300, 8491, 16, 8, 128, 0, 4096, -1) % one == 0
+    for call in ((1, 8491, 8491, 16, 8, 128, 0, 8192, 8192),    # not cached
+                 (1, 300, 4600, 16, 8, 128, 0, 4224, 4224),     # 4 KiB of keys, as one sweep
+                 (1, 8000, 16191, 16, 8, 128, 0, 8192, 8192),   # fills the GPU
+                 (1, 300, 8491, 16, 7, 128, 0, 8192, 8192),     # not a call
+                 (1, 300, 8491, 16, 8, 96, 0, 8192, 8192),
+                 (1, 300, 8491, 16, 8, 128, 4, 4, 8)):
+        assert _bytes(*call) == 0, call
+    assert _bytes(1, 300, 8491, 16, 8, 128, 0, 8192, 8192, 0.0) == 0  # exact running max
+
+
+def _whole(q, k, v, lo, mid, hi, dual):
+    B, T, H, D = q.shape
+    ot, os_ = torch.empty_like(q), torch.empty_like(q)
+    lt, ls = (torch.empty(B, H, T, device=q.device) for _ in range(2))
+    st = [_lib.strides4(x.stride()) for x in (q, k, v, ot)]
+    L = _lib.lib()
+    shape = (B, T, k.shape[1], H, k.shape[2], D)
+    stream = torch.cuda.current_stream().cuda_stream
+    if dual:
+        _lib.check(L.ttcd_dual_window_attn_kv_fwd(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), ot.data_ptr(), os_.data_ptr(),
+            lt.data_ptr(), ls.data_ptr(), *shape, *st, hi, mid, D ** -0.5, 8.0, DT[q.dtype],
+            stream))
+        return ot, os_, lt, ls
+    _lib.check(L.ttcd_band_attn_kv_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), ot.data_ptr(), lt.data_ptr(), *shape, *st, lo,
+        hi, D ** -0.5, 8.0, DT[q.dtype], stream))
+    return ot, lt
+
+
+def _close(got, want, bound, dtype, what):
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    g, w = got.float(), want.float()
+    limit = 2 * u * bound + u * w.abs() + 1e-6
+    worst = ((g - w).abs() / limit).max().item()
+    assert worst <= 1.0, (what, worst)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Tq,Tk,H,HK,D,wt,ws,dtype", [
+    (1, 1, 8192, 16, 8, 128, 8192, 4096, torch.bfloat16),     # one token, two heads a wavefront
+    (1, 300, 8491, 16, 8, 128, 8192, 4096, torch.bfloat16),
+    (2, 65, 6001, 4, 4, 128, -1, 33, torch.float16),          # full causal, near part of a tile
+    (1, 129, 9000, 15, 5, 64, 8192, 8064, torch.bfloat16),    # far part of two tiles
+    (1, 70, 5000, 4, 2, 64, 4999, 4998, torch.float16),       # far part of one key
+    (3, 7, 16390, 8, 2, 128, 16384, 8192, torch.bfloat16),
+    (1, 200, 5100, 8, 1, 64, 6000, 5100, torch.bfloat16),     # windows past the keys: no far part
+])
+@torch.inference_mode()
+def test_split_calls_match_the_whole_call(gpu, B, Tq, Tk, H, HK, D, wt, ws, dtype):
+    qf, k, v = make_qkv(batch=B, seqlen=Tk, heads=H, kv_heads=HK, head_dim=D, dtype=dtype,
+                        seed=Tq + Tk)
+    q = qf[:, Tk - Tq:]
+    k = torch.stack([k, v], 2).flatten(2, 3)[:, :, :HK]  # strided keys
+    hi = wt if wt > 0 else Tk
+    assert _bytes(B, Tq, Tk, H, HK, D, 0, ws, hi) > 0 and _bytes(B, Tq, Tk, H, HK, D, 0, hi, hi) > 0
+    mean_abs_v = window_attn(q, k, v.abs(), hi)  # sum_j p_j |v_j|, to its own rounding
+    got = fused_dual_window_attn(q, k, v, wt, ws, return_lse=True)
+    want = _whole(q, k, v, 0, ws, hi, True)
+    near = window_attn(q, k, v.abs(), ws)
+    for name, g, w, b in (("teacher", got[0], want[0], mean_abs_v), ("student", got[1], want[1], near)):
+        _close(g, w, 1.02 * b.float(), dtype, name)
+    assert (got[2] - want[2]).abs().max() <= 1e-5 and (got[3] - want[3]).abs().max() <= 1e-5
+    o, lse = window_attn(q, k, v, wt, return_lse=True)
+    wo, wl = _whole(q, k, v, 0, hi, hi, False)
+    _close(o, wo, 1.02 * mean_abs_v.float(), dtype, "window")
+    assert (lse - wl).abs().max() <= 1e-5
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_split_call_under_graph_capture(gpu):
+    qf, k, v = make_qkv(batch=1, seqlen=8300, heads=16, kv_heads=8, head_dim=128, seed=5)
+    q = qf[:, -40:].contiguous()
+    want = window_attn(q, k, v, 8192)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        out = window_attn(q, k, v, 8192)
+    for _ in range(3):
+        out.fill_(7.0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)

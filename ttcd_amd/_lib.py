@@ -33,6 +33,9 @@ EXPORTS = (
     "ttcd_band_attn_fwd",
     "ttcd_dual_window_attn_kv_fwd",
     "ttcd_band_attn_kv_fwd",
+    "ttcd_attn_kv_workspace_bytes",
+    "ttcd_dual_window_attn_kv_ws_fwd",
+    "ttcd_band_attn_kv_ws_fwd",
     "ttcd_dual_window_attn_varlen_fwd",
     "ttcd_band_attn_varlen_fwd",
     "ttcd_lse_merge_fwd",
@@ -86,6 +89,18 @@ _SIGS = {
         _i32, _i32, _i32, _i32, _i32, _i32,
         _i64x4, _i64x4, _i64x4, _i64x4,
         _i32, _i32, ctypes.c_float, ctypes.c_float, _i32, _vp]),
+    "ttcd_attn_kv_workspace_bytes": (ctypes.c_size_t, [
+        _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _i32, ctypes.c_float]),
+    "ttcd_dual_window_attn_kv_ws_fwd": (_i32, [
+        _vp, _vp, _vp, _vp, _vp, _fp, _fp,
+        _i32, _i32, _i32, _i32, _i32, _i32,
+        _i64x4, _i64x4, _i64x4, _i64x4,
+        _i32, _i32, ctypes.c_float, ctypes.c_float, _i32, _vp, ctypes.c_size_t, _vp]),
+    "ttcd_band_attn_kv_ws_fwd": (_i32, [
+        _vp, _vp, _vp, _vp, _fp,
+        _i32, _i32, _i32, _i32, _i32, _i32,
+        _i64x4, _i64x4, _i64x4, _i64x4,
+        _i32, _i32, ctypes.c_float, ctypes.c_float, _i32, _vp, ctypes.c_size_t, _vp]),
     "ttcd_dual_window_attn_varlen_fwd": (_i32, [
         _vp, _vp, _vp, _vp, _vp, _fp, _fp, _vp,
         _i32, _i32, _i32, _i32, _i32, _i32,

@@ -17,7 +17,8 @@ Windows follow flash-attention's ``(W-1, 0)`` convention: key j is visible
 to query i iff 0 <= i - j <= W - 1; a window of None or < 0 means full
 causal. The softmax scale is head_dim ** -0.5, as in the reference. All
 calls are forward-only, launch on torch's current stream, allocate only
-their outputs and never synchronise.
+their outputs (and the workspace of a split cached prefill or of the LSE
+variant) and never synchronise.
 """
 from __future__ import annotations
 
@@ -81,6 +82,18 @@ def _ready(t: torch.Tensor) -> torch.Tensor:
     return t.contiguous()
 
 
+def _split_workspace(q: torch.Tensor, Tk: int, HK: int, lo: int, mid: int, hi: int,
+                     rescale: float):
+    """(workspace or None, its bytes) for a cached prefill that the kernels would
+    split over keys (ttcd_attn_kv_workspace_bytes); the caller keeps it until
+    the call is launched."""
+    B, T, H, D = q.shape
+    if T >= Tk:
+        return None, 0
+    n = _lib.lib().ttcd_attn_kv_workspace_bytes(B, T, Tk, H, HK, D, lo, mid, hi, rescale)
+    return (torch.empty(n, dtype=torch.uint8, device=q.device) if n else None), n
+
+
 def _lse_ptr(t):
     return None if t is None else t.data_ptr()
 
@@ -103,7 +116,9 @@ def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     k / v may be longer than q (Tk > Tq, a prefill onto a populated cache):
     the queries are then the last Tq positions, flash-attention's
     bottom-right aligned causal mask, which test/test_fused_dual_attn.py:
-    275-293 asks of this call (a strict xfail for the reference kernel).
+    275-293 asks of this call (a strict xfail for the reference kernel). Few
+    queries over a long window are split over the keys, in a workspace
+    allocated here: such rows agree with the unsplit call's to rounding.
     """
     Tk = k.shape[1] if isinstance(k, torch.Tensor) and k.dim() == 4 else q.shape[1]
     if window_teacher is None or window_teacher < 0:
@@ -122,14 +137,16 @@ def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if return_lse:
         lse_t = torch.empty(B, H, T, device=q.device, dtype=torch.float32)
         lse_s = torch.empty(B, H, T, device=q.device, dtype=torch.float32)
+    wt, ws = int(min(window_teacher, 2**31 - 1)), int(min(window_student, 2**31 - 1))
+    rescale = _rescale(exact_max)
+    work, nbytes = _split_workspace(q, k.shape[1], HK, 0, ws, wt, rescale)
     L = _lib.lib()
-    _lib.check(L.ttcd_dual_window_attn_kv_fwd(
+    _lib.check(L.ttcd_dual_window_attn_kv_ws_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), ot.data_ptr(), os_.data_ptr(),
         _lse_ptr(lse_t), _lse_ptr(lse_s), B, T, k.shape[1], H, HK, D,
         _lib.strides4(q.stride()), _lib.strides4(k.stride()), _lib.strides4(v.stride()),
-        _lib.strides4(ot.stride()), int(min(window_teacher, 2**31 - 1)),
-        int(min(window_student, 2**31 - 1)), D ** -0.5, _rescale(exact_max), _DT[q.dtype],
-        _stream(q.device)))
+        _lib.strides4(ot.stride()), wt, ws, D ** -0.5, rescale, _DT[q.dtype],
+        _lse_ptr(work), nbytes, _stream(q.device)))
     if return_lse:
         return ot, os_, lse_t, lse_s
     return ot, os_
@@ -152,13 +169,16 @@ def band_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, band_lo: int, b
     q, k, v = _ready(q), _ready(k), _ready(v)
     o = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     lse = torch.empty(B, H, T, device=q.device, dtype=torch.float32) if return_lse else None
+    lo, hi = int(min(band_lo, 2**31 - 1)), int(min(band_hi, 2**31 - 1))
+    rescale = _rescale(exact_max)
+    work, nbytes = _split_workspace(q, Tk, HK, lo, hi, hi, rescale)
     L = _lib.lib()
-    _lib.check(L.ttcd_band_attn_kv_fwd(
+    _lib.check(L.ttcd_band_attn_kv_ws_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), _lse_ptr(lse),
         B, T, Tk, H, HK, D,
         _lib.strides4(q.stride()), _lib.strides4(k.stride()), _lib.strides4(v.stride()),
-        _lib.strides4(o.stride()), int(min(band_lo, 2**31 - 1)), int(min(band_hi, 2**31 - 1)),
-        D ** -0.5, _rescale(exact_max), _DT[q.dtype], _stream(q.device)))
+        _lib.strides4(o.stride()), lo, hi, D ** -0.5, rescale, _DT[q.dtype],
+        _lse_ptr(work), nbytes, _stream(q.device)))
     return (o, lse) if return_lse else o
 
 
@@ -339,5 +359,6 @@ def lse_dual_window_attn_fa3(q, k, v, window_teacher: int, window_student: int):
 
 def lse_dual_window_attn_fa3_fast(q, k, v, window_teacher: int, window_student: int):
     """profiling/lse_dual_attn.py:134-160 (two band calls + one-pass merge kernel);
-    the student output is exactly the single-window call's output."""
+    the student output is exactly the single-window call's output (to rounding
+    where that call is a cached prefill split over the keys)."""
     return lse_dual_window_attn(q, k, v, window_teacher, window_student)

@@ -159,13 +159,153 @@ static ttcd_status set_rows(ttcd::AttnArgs* a, int Tq, int Tk) {
   return TTCD_OK;
 }
 
-ttcd_status ttcd_dual_window_attn_kv_fwd(const void* q, const void* k, const void* v, void* o_t,
-                                         void* o_s, float* lse_t, float* lse_s, int B, int Tq,
-                                         int Tk, int Hq, int Hkv, int D,
-                                         const int64_t q_stride[4], const int64_t k_stride[4],
-                                         const int64_t v_stride[4], const int64_t o_stride[4],
-                                         int window_t, int window_s, float sm_scale,
-                                         float rescale_log2, ttcd_dtype dtype, void* stream) {
+// ---------------------------------------------------------------------------
+// Splitting a call over keys. A cached prefill of few query rows launches few
+// workgroups, each sweeping thousands of keys one tile after the other while
+// most CUs idle. The band of distances is then cut into parts, each swept by a
+// workgroup of its own into fp32 partials in the caller's workspace, which
+// one more launch adds up through their LSEs.
+namespace {
+
+struct SplitPlan {
+  int near_parts = 0, far_parts = 0;  // 0: not split
+  int near_step = 0, far_step = 0;
+  int parts() const { return near_parts + far_parts; }
+};
+
+constexpr size_t kSplitMaxBytes = size_t(64) << 20;
+
+size_t split_part_bytes(int B, int Tq, int Hq, int D) {
+  return (size_t)B * Tq * Hq * (D + 1) * sizeof(float);
+}
+
+// Parts of the band [lo, hi), cut at mid (mid == hi: one band; else the near
+// parts end there). The rule is a model of the call's time in us, its rates
+// fitted to an MI355X: a slot takes `alone` with its CU to itself and `busy`
+// of the CU's time when it shares it, a launch 8 to start and end, the sum 3
+// and its traffic at 5 TB/s. Over 14 shapes of 1 to 3000 queries the parts it
+// picks are within 1 % (mean) of the best of 1 to 32. A split has to promise
+// 13 %. Not split: calls whose queries are the whole sequence and sweeps of
+// up to 72 tiles, whose rows are the same bits however a prompt is cut into
+// calls, and the exact running max, which is the reference kernel's own
+// order of accumulation.
+//
+// Measured (us, whole -> split, window 8192 on 8191 cached keys), 16/8 heads
+// of 128: 1 query 127 -> 23, 64 128 -> 30, 300 128 -> 44, 600 131 -> 66, 1000
+// 131 -> 90, 2048 188 -> 173; 15/5 heads of 64: 1 query 97 -> 21, 500
+// 99 -> 40, 1000 99 -> 62.
+SplitPlan split_plan(int B, int Tq, int Tk, int Hq, int Hkv, int D, int lo, int mid, int hi,
+                     float rescale_log2) {
+  SplitPlan none, best;
+  if (Tq >= Tk || rescale_log2 <= 0.f) return none;
+  hi = hi < Tk ? hi : Tk;
+  mid = mid < hi ? mid : hi;
+  if (lo >= hi) return none;
+  const int G = Hq / Hkv, rows = ttcd::wave_rows(G), span = ttcd::wg_span_tokens(G);
+  const int sweep = (hi - lo + span - 1) / ttcd::kBlockN + 1;
+  if (sweep <= 72) return none;
+  const int64_t blocks = (Tk + span - 1) / span - (Tk - Tq) / span;
+  const int64_t nwg = (int64_t)B * Hkv * (G / (ttcd::kWaveRows / rows)) * blocks;
+  const double alone = D == 128 ? 0.95 : 0.70, busy = D == 128 ? 0.80 : 0.45;
+  const int cus = ttcd::kXcd * ttcd::kXcdCus;
+  auto model = [&](int parts) {
+    const double n = (double)((nwg * parts + cus - 1) / cus);
+    const double slots = (double)sweep / parts + (parts > 1 ? 1.5 : 0.0);
+    double t = 8.0 + slots * (alone > n * busy ? alone : n * busy);
+    if (parts > 1) t += 3.0 + 2.0 * parts * split_part_bytes(B, Tq, Hq, D) / 5e6;
+    return t;
+  };
+  double least = 0.87 * model(1);
+  for (int p = 2; p <= 16 && sweep / p >= 4; ++p) {
+    if (p * split_part_bytes(B, Tq, Hq, D) > kSplitMaxBytes) break;
+    const double t = model(p);
+    if (t >= least) continue;
+    least = t;
+    best = none;
+    auto cut = [&](int width, int parts, int* n, int* step) {
+      *step = ((width + parts - 1) / parts + ttcd::kBlockN - 1) / ttcd::kBlockN * ttcd::kBlockN;
+      *n = (width + *step - 1) / *step;
+    };
+    const int far = hi - mid;
+    int near_p = far > 0 ? (int)((int64_t)p * (mid - lo) / (hi - lo)) : p;
+    near_p = near_p < 1 ? 1 : near_p;
+    cut(mid - lo, near_p, &best.near_parts, &best.near_step);
+    if (far > 0) cut(far, p - near_p > 1 ? p - near_p : 1, &best.far_parts, &best.far_step);
+  }
+  return best;
+}
+
+// Launch the split form of a (whose o_t, o_s, lse_t, lse_s and strides are the
+// call's) in `ws`.
+ttcd_status run_split(ttcd::AttnArgs a, const SplitPlan& sp, int Tq, int D, int lo, int mid,
+                      int hi, ttcd_dtype dtype, void* ws, void* stream) {
+  const int64_t rows = (int64_t)a.B * Tq * a.Hq;
+  ttcd::CombineArgs c = {};
+  c.part = static_cast<const float*>(ws);
+  c.part_lse = c.part + rows * D * sp.parts();
+  c.o = a.o_t;
+  c.o_near = a.o_s;
+  c.lse = a.lse_t;
+  c.lse_near = a.lse_s;
+  c.B = a.B;
+  c.T = Tq;
+  c.H = a.Hq;
+  c.D = D;
+  c.parts = sp.parts();
+  c.near_parts = sp.near_parts;
+  c.sb = a.o_sb;
+  c.st = a.o_st;
+  c.sh = a.o_sh;
+  a.o_t = ws;
+  a.o_s = nullptr;
+  a.lse_t = const_cast<float*>(c.part_lse);
+  a.lse_s = nullptr;
+  a.o_sh = D;
+  a.o_st = (int64_t)a.Hq * D;
+  a.o_sb = (int64_t)Tq * a.o_st;
+  a.o_sp = rows * D;
+  a.lse_sp = rows;
+  a.parts = sp.parts();
+  a.near_parts = sp.near_parts;
+  a.near_step = sp.near_step;
+  a.far_step = sp.far_step;
+  hi = hi < a.T ? hi : a.T;
+  mid = mid < hi ? mid : hi;
+  a.near = {lo, mid};
+  a.far = {mid, hi};
+  a.sched = ttcd::make_band_schedule(a.T, lo, hi, ttcd::wave_rows(a.G));
+  hipStream_t hs = static_cast<hipStream_t>(stream);
+  ttcd_status st = from_hip(ttcd::launch_attn(a, D, elem(dtype), hs), "split attention launch");
+  if (st != TTCD_OK) return st;
+  return from_hip(ttcd::launch_attn_combine(c, elem(dtype), hs), "attention combine launch");
+}
+
+bool split_fits(const SplitPlan& sp, const void* ws, size_t bytes, int B, int Tq, int Hq, int D) {
+  return sp.parts() > 1 && ws != nullptr && (reinterpret_cast<uintptr_t>(ws) & 15u) == 0 &&
+         bytes >= sp.parts() * split_part_bytes(B, Tq, Hq, D);
+}
+
+}  // namespace
+
+size_t ttcd_attn_kv_workspace_bytes(int B, int Tq, int Tk, int Hq, int Hkv, int D, int band_lo,
+                                    int band_mid, int band_hi, float rescale_log2) {
+  if (B < 1 || Tq < 1 || Tq > Tk || Hkv < 1 || Hq < Hkv || Hq % Hkv != 0 ||
+      (D != 64 && D != 128) || band_lo < 0)
+    return 0;
+  if (band_hi < 0) band_hi = Tk;
+  if (band_mid < 0) band_mid = band_hi;
+  if (band_mid <= band_lo || band_mid > band_hi) return 0;
+  const SplitPlan sp =
+      split_plan(B, Tq, Tk, Hq, Hkv, D, band_lo, band_mid, band_hi, rescale_log2);
+  return sp.parts() > 1 ? sp.parts() * split_part_bytes(B, Tq, Hq, D) : 0;
+}
+
+ttcd_status ttcd_dual_window_attn_kv_ws_fwd(
+    const void* q, const void* k, const void* v, void* o_t, void* o_s, float* lse_t, float* lse_s,
+    int B, int Tq, int Tk, int Hq, int Hkv, int D, const int64_t q_stride[4],
+    const int64_t k_stride[4], const int64_t v_stride[4], const int64_t o_stride[4], int window_t,
+    int window_s, float sm_scale, float rescale_log2, ttcd_dtype dtype, void* workspace,
+    size_t workspace_bytes, void* stream) {
   ttcd_status st =
       check_attn(q, k, v, o_t, B, Tk, Hq, Hkv, D, q_stride, k_stride, v_stride, o_stride, dtype);
   if (st == TTCD_OK) st = check_rescale(rescale_log2, dtype);
@@ -188,9 +328,28 @@ ttcd_status ttcd_dual_window_attn_kv_fwd(const void* q, const void* k, const voi
   a.lse_t = lse_t;
   a.lse_s = lse_s;
   a.rescale_log2 = rescale_log2;
+  if (workspace_bytes > 0) {
+    const SplitPlan sp =
+        split_plan(B, Tq, Tk, Hq, Hkv, D, 0, window_s, window_t, rescale_log2);
+    if (split_fits(sp, workspace, workspace_bytes, B, Tq, Hq, D))
+      return run_split(a, sp, Tq, D, 0, window_s, window_t, dtype, workspace, stream);
+  }
   a.sched = ttcd::make_dual_schedule(Tk, window_s, window_t, ttcd::wave_rows(a.G));
   return from_hip(ttcd::launch_attn(a, D, elem(dtype), static_cast<hipStream_t>(stream)),
                   "dual-window attention launch");
+}
+
+ttcd_status ttcd_dual_window_attn_kv_fwd(const void* q, const void* k, const void* v, void* o_t,
+                                         void* o_s, float* lse_t, float* lse_s, int B, int Tq,
+                                         int Tk, int Hq, int Hkv, int D,
+                                         const int64_t q_stride[4], const int64_t k_stride[4],
+                                         const int64_t v_stride[4], const int64_t o_stride[4],
+                                         int window_t, int window_s, float sm_scale,
+                                         float rescale_log2, ttcd_dtype dtype, void* stream) {
+  return ttcd_dual_window_attn_kv_ws_fwd(q, k, v, o_t, o_s, lse_t, lse_s, B, Tq, Tk, Hq, Hkv, D,
+                                         q_stride, k_stride, v_stride, o_stride, window_t,
+                                         window_s, sm_scale, rescale_log2, dtype, nullptr, 0,
+                                         stream);
 }
 
 ttcd_status ttcd_dual_window_attn_fwd(const void* q, const void* k, const void* v, void* o_t,
@@ -204,12 +363,13 @@ ttcd_status ttcd_dual_window_attn_fwd(const void* q, const void* k, const void* 
                                       sm_scale, ttcd::kDefaultRescaleLog2, dtype, stream);
 }
 
-ttcd_status ttcd_band_attn_kv_fwd(const void* q, const void* k, const void* v, void* o,
-                                  float* lse, int B, int Tq, int Tk, int Hq, int Hkv, int D,
-                                  const int64_t q_stride[4], const int64_t k_stride[4],
-                                  const int64_t v_stride[4], const int64_t o_stride[4],
-                                  int band_lo, int band_hi, float sm_scale, float rescale_log2,
-                                  ttcd_dtype dtype, void* stream) {
+ttcd_status ttcd_band_attn_kv_ws_fwd(const void* q, const void* k, const void* v, void* o,
+                                     float* lse, int B, int Tq, int Tk, int Hq, int Hkv, int D,
+                                     const int64_t q_stride[4], const int64_t k_stride[4],
+                                     const int64_t v_stride[4], const int64_t o_stride[4],
+                                     int band_lo, int band_hi, float sm_scale,
+                                     float rescale_log2, ttcd_dtype dtype, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
   ttcd_status st =
       check_attn(q, k, v, o, B, Tk, Hq, Hkv, D, q_stride, k_stride, v_stride, o_stride, dtype);
   if (st == TTCD_OK) st = check_rescale(rescale_log2, dtype);
@@ -226,9 +386,26 @@ ttcd_status ttcd_band_attn_kv_fwd(const void* q, const void* k, const void* v, v
   a.o_t = o;
   a.lse_t = lse;
   a.rescale_log2 = rescale_log2;
+  if (workspace_bytes > 0) {
+    const SplitPlan sp =
+        split_plan(B, Tq, Tk, Hq, Hkv, D, band_lo, band_hi, band_hi, rescale_log2);
+    if (split_fits(sp, workspace, workspace_bytes, B, Tq, Hq, D))
+      return run_split(a, sp, Tq, D, band_lo, band_hi, band_hi, dtype, workspace, stream);
+  }
   a.sched = ttcd::make_band_schedule(Tk, band_lo, band_hi, ttcd::wave_rows(a.G));
   return from_hip(ttcd::launch_attn(a, D, elem(dtype), static_cast<hipStream_t>(stream)),
                   "band attention launch");
+}
+
+ttcd_status ttcd_band_attn_kv_fwd(const void* q, const void* k, const void* v, void* o,
+                                  float* lse, int B, int Tq, int Tk, int Hq, int Hkv, int D,
+                                  const int64_t q_stride[4], const int64_t k_stride[4],
+                                  const int64_t v_stride[4], const int64_t o_stride[4],
+                                  int band_lo, int band_hi, float sm_scale, float rescale_log2,
+                                  ttcd_dtype dtype, void* stream) {
+  return ttcd_band_attn_kv_ws_fwd(q, k, v, o, lse, B, Tq, Tk, Hq, Hkv, D, q_stride, k_stride,
+                                  v_stride, o_stride, band_lo, band_hi, sm_scale, rescale_log2,
+                                  dtype, nullptr, 0, stream);
 }
 
 ttcd_status ttcd_band_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse,

@@ -50,6 +50,9 @@
 //     128, windows 8192 / 4096: 1782 -> 1754 us), 5 % at windows 2048 / 1024
 //     (T = 5003, 173 -> 165 us), 8 % at 512 / 256 (T = 2048, 4/2 heads of
 //     64, 15.4 -> 14.1 us).
+//   * A cached prefill of few queries over many keys may be split over the
+//     keys (PART): a workgroup folds one sub-band of distances and writes fp32
+//     partials, which merge.hip adds up (api.hip: split_plan, with figures).
 //   * Packed sequences (cu_seqlens): each workgroup builds its sequence's
 //     schedule from the sequence length, with every bound clamped to the
 //     packed tensors.
@@ -92,6 +95,7 @@ namespace ttcd {
 namespace {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -399,6 +403,31 @@ __device__ __forceinline__ void emit(const f32x16 (&o)[Geo<D>::DT], float m, flo
   }
 }
 
+// One part of a call split over keys: the normalised fp32 output and its LSE.
+template <int D>
+__device__ __forceinline__ void emit_part(const f32x16 (&o)[Geo<D>::DT], float m, float l,
+                                          float c, float* out, int64_t o_st, float* lse,
+                                          int qrow, int T_, int q_off, int lane) {
+  const float lt = xhalf_sum(l);
+  const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+  if (qrow >= T_ || qrow < q_off) return;
+  const int half = lane >> 5;
+  float* dst = out + (int64_t)(qrow - q_off) * o_st + half * 4;
+#pragma unroll
+  for (int dt = 0; dt < Geo<D>::DT; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = o[dt][4 * g + e] * inv;
+      *reinterpret_cast<f32x4*>(dst + dt * 32 + 8 * g) = w;
+    }
+  if (half == 0) {
+    const float mc = (m == -INFINITY) ? 0.f : m * c;
+    lse[qrow - q_off] = lt > 0.f ? mc * 0.69314718055994531f + logf(lt) : -INFINITY;
+  }
+}
+
 // Everything the slot body needs besides the per-slot registers.
 template <int D, typename T>
 struct Ctx {
@@ -676,7 +705,9 @@ constexpr int waves_per_simd() {
   return D == 64 ? TTCD_D64_WAVES : 2;
 }
 
-template <int D, typename T, bool DUAL, bool LAZY>
+// PART: the workgroup folds one sub-band of a call split over keys (AttnArgs)
+// and writes fp32 partials, for attn_combine_kernel to add up.
+template <int D, typename T, bool DUAL, bool LAZY, bool PART = false>
 __global__ __attribute__((amdgpu_flat_work_group_size(kWaves * 64, kWaves * 64),
                           amdgpu_waves_per_eu(waves_per_simd<D>(), waves_per_simd<D>())))
 void attn_fwd_kernel(AttnArgs a) {
@@ -703,6 +734,11 @@ void attn_fwd_kernel(AttnArgs a) {
   int pair, qb, g;
   if (!a.map.locate((int)__builtin_amdgcn_workgroup_id_x(), &pair, &qb, &g)) return;
   qb += a.qb0;
+  int part = 0;
+  if constexpr (PART) {
+    part = a.pairs.quot(pair);
+    pair -= part * (int)a.pairs.d;
+  }
   const int b = a.hkv.quot(pair);
   const int hk = pair - b * a.Hkv;
   const int h = hk * a.G + g * hpw;  // the wavefront's first query head
@@ -719,7 +755,15 @@ void attn_fwd_kernel(AttnArgs a) {
   int T_ = a.T;
   int64_t row0 = 0;
   Schedule sc = a.sched;
-  if (a.cu_seqlens != nullptr) {
+  if constexpr (PART) {
+    const bool far = part >= a.near_parts;
+    const Band whole = far ? a.far : a.near;
+    const int step = far ? a.far_step : a.near_step;
+    sc.p1.lo = whole.lo + (far ? part - a.near_parts : part) * step;
+    sc.p1.hi = min(sc.p1.lo + step, whole.hi);
+    sc.p2.lo = sc.p2.hi = sc.p1.hi;
+  }
+  if (!PART && a.cu_seqlens != nullptr) {
     const int c0 = __builtin_amdgcn_readfirstlane(a.cu_seqlens[b]);
     const int c1 = __builtin_amdgcn_readfirstlane(a.cu_seqlens[b + 1]);
     const int s0 = min(max(c0, 0), a.total);
@@ -980,6 +1024,13 @@ void attn_fwd_kernel(AttnArgs a) {
     if (k + 1 < nslot) step(s1, s0, pb, pa, k + 1);
   }
 
+  if constexpr (PART) {
+    if (wave_valid)
+      emit_part<D>(o, m, l, x.c, static_cast<float*>(a.o_t) + part * a.o_sp + o_base + o_dh(),
+                   a.o_st, a.lse_t + part * a.lse_sp + lse_base + lse_dh(), x.qrow, T_, q_off,
+                   lane);
+    return;
+  }
   if (wave_valid) {
     if (DUAL && !emitted_s) {
       T* os = static_cast<T*>(a.o_s) + o_base + o_dh();
@@ -1014,8 +1065,22 @@ hipError_t launch_typed(const AttnArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// A call split over keys: part-major K/V heads, lazy slots (or D = 64's own).
+template <int D, typename T>
+hipError_t launch_parts(const AttnArgs& a, hipStream_t stream) {
+  AttnArgs args = a;
+  args.map = make_block_map(a.B * a.Hkv * a.parts, a.nqb,
+                            a.G / (kWaveRows / a.sched.rows), false);
+  args.hkv = make_fast_div(a.Hkv);
+  args.pairs = make_fast_div(a.B * a.Hkv);
+  hipLaunchKernelGGL((attn_fwd_kernel<D, T, false, D == 128, true>), dim3(args.map.launched()),
+                     dim3(kWaves * 64), 0, stream, args);
+  return hipGetLastError();
+}
+
 template <int D, typename T>
 hipError_t launch_dual_or_band(const AttnArgs& a, hipStream_t stream) {
+  if (a.parts > 0) return launch_parts<D, T>(a, stream);
   return a.sched.dual ? launch_typed<D, T, true>(a, stream) : launch_typed<D, T, false>(a, stream);
 }
 

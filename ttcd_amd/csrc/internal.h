@@ -43,6 +43,15 @@ struct AttnArgs {
   const int* cu_seqlens;
   int total;
   int win_a, win_b;
+  // A call split over keys (parts > 0): part p of a workgroup's rows folds a
+  // sub-band of distances, [lo + p * step, ..) below `mid` for the near_parts
+  // first ones and on from mid for the rest, and writes fp32 outputs and LSEs
+  // to o_t / lse_t, o_sp / lse_sp elements from one part to the next.
+  int parts, near_parts;
+  int near_step, far_step;
+  Band near, far;  // [lo, mid), [mid, hi)
+  FastDiv pairs;   // division by B * Hkv
+  int64_t o_sp, lse_sp;
 };
 
 // Default lazy-rescale threshold (log2 units) of the attention entry points
@@ -144,5 +153,19 @@ struct MergeArgs {
   int64_t f_sb, f_st, f_sh;
 };
 hipError_t launch_lse_merge(const MergeArgs& a, Elem dtype, hipStream_t stream);
+
+// The outputs of a call split over keys from its parts (merge.hip): o / lse
+// from all of them, and o_near / lse_near (optional) from the near_parts first.
+struct CombineArgs {
+  const float* part;      // (parts, B, T, H, D)
+  const float* part_lse;  // (parts, B, H, T)
+  void* o;
+  void* o_near;
+  float* lse;             // (B, H, T), or null
+  float* lse_near;
+  int B, T, H, D, parts, near_parts;
+  int64_t sb, st, sh;     // strides of o and o_near
+};
+hipError_t launch_attn_combine(const CombineArgs& a, Elem dtype, hipStream_t stream);
 
 }  // namespace ttcd

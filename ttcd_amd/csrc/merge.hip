@@ -10,6 +10,11 @@
 // own (the LSE variant keeps it in a chunk-sized scratch). HBM-bound
 // elementwise pass: each thread moves 16 bytes of each operand with
 // coalesced vector accesses, non-temporal loads for the partials (read once).
+//
+// attn_combine_kernel is the same identity for an attention call split over
+// keys into any number of fp32 parts (attn.hip, PART): weights exp(lse_p - m)
+// with m the row's largest LSE, one division and one rounding at the end; the
+// near parts' running sums give the student's output on the way.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -20,6 +25,7 @@ namespace ttcd {
 namespace {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 template <typename T>
 union P8 {
@@ -83,7 +89,69 @@ hipError_t launch_typed(const MergeArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// One thread: 8 elements of one row. The parts' LSEs of a row are shared by its
+// D / 8 threads (one cache line); their outputs are read once, 32 bytes a
+// thread and part.
+template <typename T>
+__global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs a) {
+  const int ng = a.D / 8;
+  const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t rows = (int64_t)a.B * a.T * a.H;
+  if (gid >= rows * ng) return;
+  const int64_t row = gid / ng;  // (b, t, h)
+  const int dg = (int)(gid - row * ng);
+  const int64_t bt = row / a.H;
+  const int h = (int)(row - bt * a.H);
+  const int b = (int)(bt / a.T);
+  const int t = (int)(bt - (int64_t)b * a.T);
+  const int64_t li = ((int64_t)b * a.H + h) * a.T + t;
+  const float* src = a.part + row * a.D + dg * 8;
+  const int64_t off = b * a.sb + t * a.st + h * a.sh + dg * 8;
+
+  float m = -INFINITY;
+  for (int p = 0; p < a.parts; ++p) m = fmaxf(m, a.part_lse[p * rows + li]);
+  const float ref = m == -INFINITY ? 0.f : m;
+  float acc[8], sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  auto emit = [&](void* o, float* lse) {
+    const float inv = sum > 0.f ? 1.0f / sum : 0.f;
+    P8<T> out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out.e[e] = static_cast<T>(acc[e] * inv);
+    *reinterpret_cast<u32x4*>(static_cast<T*>(o) + off) = out.raw;
+    if (lse != nullptr && dg == 0) lse[li] = sum > 0.f ? ref + logf(sum) : -INFINITY;
+  };
+  for (int p = 0; p < a.parts; ++p) {
+    if (p == a.near_parts && a.o_near != nullptr) emit(a.o_near, a.lse_near);
+    const float w = expf(a.part_lse[p * rows + li] - ref);
+    const f32x4* v = reinterpret_cast<const f32x4*>(src + p * rows * a.D);
+    const f32x4 lo = __builtin_nontemporal_load(v), hi = __builtin_nontemporal_load(v + 1);
+    sum += w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      acc[e] = fmaf(lo[e], w, acc[e]);
+      acc[4 + e] = fmaf(hi[e], w, acc[4 + e]);
+    }
+  }
+  if (a.near_parts == a.parts && a.o_near != nullptr) emit(a.o_near, a.lse_near);
+  emit(a.o, a.lse);
+}
+
+template <typename T>
+hipError_t launch_combine(const CombineArgs& a, hipStream_t stream) {
+  const int64_t total = (int64_t)a.B * a.T * a.H * (a.D / 8);
+  const int64_t blocks = (total + 255) / 256;
+  hipLaunchKernelGGL((attn_combine_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
 }  // namespace
+
+hipError_t launch_attn_combine(const CombineArgs& a, Elem dtype, hipStream_t stream) {
+  return dtype == Elem::BF16 ? launch_combine<__bf16>(a, stream)
+                             : launch_combine<_Float16>(a, stream);
+}
 
 hipError_t launch_lse_merge(const MergeArgs& a, Elem dtype, hipStream_t stream) {
   return dtype == Elem::BF16 ? launch_typed<__bf16>(a, stream) : launch_typed<_Float16>(a, stream);
