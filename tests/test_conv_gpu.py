@@ -90,3 +90,33 @@ def test_random_shapes_bitwise_vs_oracle(gpu, i):
     x = torch.randn(*shape, generator=g).to(xdt)
     w = torch.randn(shape[-1], K, generator=g).to(wdt)
     assert _bits_equal(_run(x, w), conv_ref.dwconv_c(x, w)), f"case {i}"
+
+
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("N,C,D,K,shift", [
+    (2, 70, 8, 5, 1), (1, 65, 9, 5, 0), (3, 64, 15, 8, 0), (1, 17, 135, 3, 3), (2, 33, 128, 5, 1),
+    (1, 40, 7, 5, 0), (2, 9, 64, 9, 0), (1, 100, 131, 16, 0), (1, 8, 33, 64, 1),
+    # above 2^19 outputs, where the vector kernels start
+    (4, 130, 1027, 4, 0), (3000, 13, 15, 5, 0), (1000, 70, 9, 8, 0), (1, 525, 1001, 16, 3),
+    (600, 70, 16, 7, 0), (40, 1000, 24, 1, 0), (520, 65, 24, 8, 0), (3000, 17, 24, 2, 0),
+    (20, 3, 9000, 5, 0), (70, 1000, 8, 5, 1), (5, 1700, 64, 9, 0), (9, 8, 8191, 64, 1), (80000, 1, 7, 3, 0)])
+@torch.inference_mode()
+def test_rows_off_alignment_bitwise_vs_oracle(gpu, N, C, D, K, shift, xdt):
+    """Rows that are not 16-byte aligned (ragged D, base address off by elements),
+    a last group of one to all but one own channels, taps past the register
+    window, and nothing written past the tensor."""
+    g = torch.Generator().manual_seed(N * C + D + K)
+    n = N * C * D
+    flat = torch.randn(n + shift, generator=g).to(xdt)
+    x = flat[shift:].view(N, C, D)
+    w = torch.randn(D, K, generator=g).to(xdt)
+    xg, wg = flat.cuda()[shift:].view(N, C, D), w.cuda()
+    yg = torch.full((n + shift + 64,), 3.0, dtype=xdt, device=gpu)
+    from ttcd_amd import _lib
+    dt = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}[xdt]
+    _lib.check(_lib.lib().ttcd_causal_dwconv_chunked_fwd(
+        xg.data_ptr(), wg.data_ptr(), yg[shift:].data_ptr(), N, C, D, K, dt, dt,
+        torch.cuda.current_stream().cuda_stream))
+    y = yg.cpu()
+    assert (y[:shift] == 3.0).all() and (y[shift + n:] == 3.0).all()
+    assert _bits_equal(y[shift:shift + n].view(N, C, D), conv_ref.dwconv_c(x, w))
