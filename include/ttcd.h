@@ -451,6 +451,11 @@ ttcd_status ttcd_ttt_features_tokens_fwd(const void* gu_t, int64_t t_rows,
 ttcd_status ttcd_ttt_proj_beta_t_fwd(const void* pd, int64_t pd_stride, const void* beta,
                                     int64_t beta_batch_stride, void* pdt, int B, int nupd,
                                     int chunk, int H, ttcd_dtype dtype, void* stream);
+/* beta[b * rows + r] = sigmoid(t[b * t_rows + r] . b_proj), the per-token
+ * learning rate (:72-74): the product summed in fp32 and rounded to dtype, its
+ * sigmoid rounded again. t rows are H contiguous elements, H % 8 == 0. */
+ttcd_status ttcd_ttt_beta_fwd(const void* t, int64_t t_rows, const void* b_proj, void* beta,
+                              int B, int rows, int H, ttcd_dtype dtype, void* stream);
 ttcd_status ttcd_ttt_scan_fwd(const void* dw, const void* w_cur, float lr, void* steps_t,
                               void* w_next, int nupd, int nsteps, int H, int inter,
                               ttcd_dtype dtype, void* stream);

@@ -66,3 +66,58 @@ def test_features_of_tokens_equal_the_padded_pass(gpu, B, tokens, C, I, ct, cs):
     wz, wzh, wdiff = ttt.ttt_features(pad[0], pad[1], w_t, w_s, B, nchunk, C)
     assert torch.equal(z, wz.view(B, nchunk * C, I)) and torch.equal(diff, wdiff)
     assert torch.equal(zh, wzh.view(B, nchunk * C, I)[:, :upd].reshape(-1, I))
+
+
+@pytest.mark.parametrize("B,L,rows,H,dtype", [
+    (1, 5, 5, 8, torch.bfloat16), (2, 300, 257, 1024, torch.bfloat16),
+    (3, 66, 64, 520, torch.float16), (1, 1030, 1023, 2048, torch.bfloat16)])
+@torch.inference_mode()
+def test_beta_is_the_rounded_sigmoid_of_the_rounded_product(gpu, B, L, rows, H, dtype):
+    """Against 64 bits. The fp32 sum of H products is off by at most H 2^-24 of
+    their magnitudes' sum, which can move the rounded product by one unit u; the
+    sigmoid passes on at most a quarter of that and rounds once more."""
+    g = torch.Generator().manual_seed(H + rows)
+    t = torch.randn(B, L, H, generator=g).to(dtype).cuda()
+    w = (torch.randn(H, generator=g) * H ** -0.5).to(dtype).cuda()
+    got = ttt._beta(t, w, rows).double()
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    dot = t[:, :rows].double() @ w.double()
+    size = t[:, :rows].double().abs() @ w.double().abs()
+    want = torch.sigmoid(dot)
+    limit = (u * dot.abs() + H * 2.0 ** -24 * size) / 4 + u * want
+    assert got.shape == (B, rows) and ((got - want).abs() <= limit).all()
+
+
+@pytest.mark.parametrize("B,K,C,H,dtype,with_beta", [
+    (1, 2, 8, 8, torch.bfloat16, True), (2, 3, 72, 136, torch.float16, True),
+    (1, 1, 64, 64, torch.bfloat16, False), (1, 2, 200, 1032, torch.bfloat16, True)])
+@torch.inference_mode()
+def test_transposed_update_on_whole_groups(gpu, B, K, C, H, dtype, with_beta):
+    """16-byte rows and columns at the edges of the 64 x 64 tiles, bit for bit torch's
+    multiply; the row stride wider than a row."""
+    g = torch.Generator().manual_seed(C + H)
+    pd = torch.randn(B * K * C, H + 16, generator=g).to(dtype).cuda()[:, :H]
+    beta = torch.rand(B, K, C, generator=g).to(dtype).cuda() if with_beta else None
+    got = ttt.proj_beta_t(pd, beta, B, K, C)
+    want = pd.reshape(B, K, C, H)
+    want = want * beta[..., None] if with_beta else want
+    assert torch.equal(got, want.transpose(2, 3).reshape(B * K, H, C))
+
+
+@pytest.mark.parametrize("nupd,nsteps,H,I,want_next", [
+    (0, 1, 8, 8, False), (1, 2, 72, 136, True), (5, 4, 64, 64, True), (3, 4, 136, 1032, False)])
+@torch.inference_mode()
+def test_scan_on_whole_groups(gpu, nupd, nsteps, H, I, want_next):
+    """Tile edges of the 16-byte scan, bit for bit torch's rounded steps."""
+    g = torch.Generator().manual_seed(H + I)
+    w = torch.randn(H, I, generator=g).to(torch.bfloat16).cuda()
+    dw = torch.randn(nupd, H, I, generator=g).to(torch.bfloat16).cuda() if nupd else None
+    steps, nxt = ttt.scan_steps(dw, w, 0.3, nsteps, want_next)
+    lr = torch.tensor(0.3, dtype=torch.bfloat16, device=gpu)
+    acc, ws = torch.zeros_like(w), [w]
+    for j in range(nupd):
+        acc = acc + dw[j]
+        ws.append(w + lr * acc)
+    for s_ in range(nsteps):
+        assert torch.equal(steps[s_], ws[s_].t()), s_
+    assert nxt is None if not want_next else torch.equal(nxt, ws[nupd])

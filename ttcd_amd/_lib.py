@@ -53,6 +53,7 @@ EXPORTS = (
     "ttcd_ttt_features_fwd",
     "ttcd_ttt_features_tokens_fwd",
     "ttcd_ttt_proj_beta_t_fwd",
+    "ttcd_ttt_beta_fwd",
     "ttcd_ttt_scan_fwd",
     "ttcd_attn_schedule_coverage",
     "ttcd_attn_block_coverage",
@@ -149,6 +150,7 @@ _SIGS = {
         _i32, _i32, _i32, _i32, _i32, _vp]),
     "ttcd_ttt_proj_beta_t_fwd": (_i32, [
         _vp, _i64, _vp, _i64, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
+    "ttcd_ttt_beta_fwd": (_i32, [_vp, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _vp]),
     "ttcd_ttt_scan_fwd": (_i32, [
         _vp, _vp, ctypes.c_float, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "ttcd_attn_schedule_coverage": (_i32, [

@@ -1062,6 +1062,20 @@ ttcd_status ttcd_ttt_proj_beta_t_fwd(const void* pd, int64_t pd_stride, const vo
                   "ttt pd*beta launch");
 }
 
+ttcd_status ttcd_ttt_beta_fwd(const void* t, int64_t t_rows, const void* b_proj, void* beta,
+                              int B, int rows, int H, ttcd_dtype dtype, void* stream) {
+  if (!t || !b_proj || !beta) return fail(TTCD_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if (B < 1 || rows < 1 || H < 1 || t_rows < rows)
+    return fail(TTCD_ERR_INVALID_ARGUMENT, "need B, rows, H >= 1 and t_rows >= rows");
+  if (dtype != TTCD_DTYPE_BF16 && dtype != TTCD_DTYPE_F16)
+    return fail(TTCD_ERR_UNSUPPORTED, "dtype must be bf16 or f16");
+  if (H % 8 != 0 || !aligned16(t) || !aligned16(b_proj))
+    return fail(TTCD_ERR_UNSUPPORTED, "H must be a multiple of 8 and t, b_proj 16-byte aligned");
+  ttcd::TttBetaArgs a{t, t_rows, b_proj, beta, B, rows, H};
+  return from_hip(ttcd::launch_ttt_beta(a, elem(dtype), static_cast<hipStream_t>(stream)),
+                  "ttt beta launch");
+}
+
 ttcd_status ttcd_ttt_scan_fwd(const void* dw, const void* w_cur, float lr, void* steps_t,
                               void* w_next, int nupd, int nsteps, int H, int inter,
                               ttcd_dtype dtype, void* stream) {

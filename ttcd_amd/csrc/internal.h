@@ -127,6 +127,13 @@ struct TttProjBetaArgs {
   void* pdt;           // (B * nupd, H, C) contiguous
   int B, nupd, C, H;
 };
+struct TttBetaArgs {
+  const void* t;       // rows of H; sequence b's start at row b * t_rows
+  int64_t t_rows;
+  const void* w;       // (H)
+  void* beta;          // (B, rows) contiguous
+  int B, rows, H;
+};
 struct TttScanArgs {
   const void* dw;      // (nupd, H, I) contiguous
   const void* w_cur;   // (H, I) contiguous
@@ -136,6 +143,7 @@ struct TttScanArgs {
   int nupd, nsteps, H, I;
 };
 hipError_t launch_ttt_proj_beta_t(const TttProjBetaArgs& a, Elem dtype, hipStream_t stream);
+hipError_t launch_ttt_beta(const TttBetaArgs& a, Elem dtype, hipStream_t stream);
 hipError_t launch_ttt_scan(const TttScanArgs& a, Elem dtype, hipStream_t stream);
 
 hipError_t launch_dwconv(const void* x, const void* w, void* y, int64_t N, int C,

@@ -52,7 +52,11 @@
 // tensor), cs_j = lr * sum_j rounded, W_step = W_cur + cs rounded, and the
 // next group's W_cur; it writes every chunk's W_step transposed, (step, I, H),
 // so the per-chunk output GEMMs z_c W_step^T (:161-165) are one batched GEMM
-// on contiguous operands as well. Both transpose through 64 x 64 LDS tiles.
+// on contiguous operands as well. Both transpose through 64 x 64 LDS tiles, in
+// 16-byte accesses where the rows allow it (20480 x 1024 pd 39 -> 15 us; 5
+// updates of 1024 x 3072 48 -> 16 us) and else by single elements.
+// ttt_beta_kernel is the learning rate itself, sigmoid(t . b_proj): one read of
+// t (20480 x 1024: 14 us; torch's product and sigmoid 23).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -455,17 +459,216 @@ __global__ __launch_bounds__(256) void ttt_scan_kernel(TttScanArgs a) {
   }
 }
 
+// The same two passes on rows of whole 16-byte groups. A thread moves 8
+// neighbouring elements of two rows of a 64 x 64 tile at a time; the tile is
+// kept transposed in LDS as 16-bit values, at a pitch of 33 words (the 8
+// threads of a row then write 8 words apart, and a column is read back as
+// words).
+constexpr int kTileWords = kTile / 2 + 1;
+
+template <typename T>
+struct TileT {
+  uint32_t w[kTile * kTileWords];
+
+  // element (row, col + e) of the tile, e = 0..7
+  __device__ void put(int row, int col, const V8<T>& v) {
+    T* p = reinterpret_cast<T*>(w);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) p[(col + e) * 2 * kTileWords + row] = v.e[e];
+  }
+  // elements (row .. row + 7, col)
+  __device__ V8<T> get(int row, int col) const {
+    V8<T> v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v.raw[q] = w[col * kTileWords + row / 2 + q];
+    return v;
+  }
+};
+
+template <typename T>
+__global__ __launch_bounds__(256) void ttt_pd_beta_t_vec_kernel(TttProjBetaArgs a) {
+  __shared__ TileT<T> tile;
+  const int row = threadIdx.x / 8, col = (threadIdx.x % 8) * 8;
+  const int h0 = blockIdx.x * kTile, t0 = blockIdx.y * kTile, bk = blockIdx.z;
+  const int b = bk / a.nupd, c = bk % a.nupd;
+  const T* pd = static_cast<const T*>(a.pd) + (int64_t)bk * a.C * a.pd_stride;
+  const T* beta = a.beta ? static_cast<const T*>(a.beta) + b * a.beta_sb + (int64_t)c * a.C
+                         : nullptr;
+  V8<T> v[2];
+  float be[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int t = min(t0 + row + 32 * r, a.C - 1), h = min(h0 + col, a.H - 8);
+    v[r].raw = __builtin_nontemporal_load(
+        reinterpret_cast<const u32x4*>(pd + (int64_t)t * a.pd_stride + h));
+    be[r] = beta ? static_cast<float>(beta[t]) : 1.f;
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    if (beta) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[r].e[e] = round_to<T>(static_cast<float>(v[r].e[e]) * be[r]);
+    }
+    tile.put(row + 32 * r, col, v[r]);
+  }
+  __syncthreads();
+  T* out = static_cast<T*>(a.pdt) + (int64_t)bk * a.H * a.C;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int h = h0 + row + 32 * r, t = t0 + col;
+    if (h < a.H && t < a.C)
+      *reinterpret_cast<u32x4*>(out + (int64_t)h * a.C + t) = tile.get(col, row + 32 * r).raw;
+  }
+}
+
+// One step's chunk update is requested while the one before it is folded, and
+// two tiles alternate, so a step has one barrier.
+template <typename T>
+__global__ __launch_bounds__(256) void ttt_scan_vec_kernel(TttScanArgs a) {
+  __shared__ TileT<T> tile[2];
+  const int row = threadIdx.x / 8, col = (threadIdx.x % 8) * 8;
+  const int i0 = blockIdx.x * kTile, h0 = blockIdx.y * kTile;
+  const int64_t HI = (int64_t)a.H * a.I;
+  int64_t off[2];
+  bool ok[2];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const int h = h0 + row + 32 * r, i = i0 + col;
+    ok[r] = h < a.H && i < a.I;
+    off[r] = (int64_t)min(h, a.H - 1) * a.I + min(i, a.I - 8);
+  }
+  auto load = [&](const void* p, int64_t at) {
+    V8<T> v;
+    v.raw = __builtin_nontemporal_load(
+        reinterpret_cast<const u32x4*>(static_cast<const T*>(p) + at));
+    return v;
+  };
+  T* steps = static_cast<T*>(a.steps_t);
+  auto store_t = [&](const V8<T> (&v)[2], int step) {
+    TileT<T>& tl = tile[step & 1];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) tl.put(row + 32 * r, col, v[r]);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const int i = i0 + row + 32 * r, h = h0 + col;
+      if (i < a.I && h < a.H)
+        *reinterpret_cast<u32x4*>(steps + step * HI + (int64_t)i * a.H + h) =
+            tl.get(col, row + 32 * r).raw;
+    }
+  };
+  V8<T> w[2], ws[2], d[2];
+  float acc[2][8];
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    w[r] = ws[r] = load(a.w_cur, off[r]);
+    if (a.nupd > 0) d[r] = load(a.dw, off[r]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
+  }
+  store_t(w, 0);  // step 0: W_cur
+  for (int j = 0; j < a.nupd; ++j) {
+    V8<T> nx[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      nx[r] = load(a.dw, (j + 1 < a.nupd ? (j + 1) * HI : 0) + off[r]);
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        // the running sum stored, lr * sum, W_cur + cs_j, each rounded
+        acc[r][e] =
+            static_cast<float>(round_to<T>(acc[r][e] + static_cast<float>(d[r].e[e])));
+        const float cs = static_cast<float>(round_to<T>(a.lr * acc[r][e]));
+        ws[r].e[e] = round_to<T>(static_cast<float>(w[r].e[e]) + cs);
+      }
+    if (j + 1 < a.nsteps) store_t(ws, j + 1);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) d[r] = nx[r];
+  }
+  if (a.w_next != nullptr) {
+    T* wn = static_cast<T*>(a.w_next);
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+      if (ok[r]) *reinterpret_cast<u32x4*>(wn + off[r]) = ws[r].raw;
+  }
+}
+
+// beta = sigmoid(t . b_proj) per token: a wavefront takes four rows, so that a
+// lane has four row loads in flight for one of the weight.
+constexpr int kBetaRows = 4;
+
+template <typename T>
+__global__ __launch_bounds__(256) void ttt_beta_kernel(TttBetaArgs a) {
+  const int lane = threadIdx.x & 63;
+  const int64_t r0 = (((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6) * kBetaRows;
+  const int64_t total = (int64_t)a.B * a.rows;
+  if (r0 >= total) return;  // whole wavefronts leave
+  const T* src[kBetaRows];
+  float acc[kBetaRows];
+#pragma unroll
+  for (int r = 0; r < kBetaRows; ++r) {
+    const int64_t row = min(r0 + r, total - 1);
+    const int64_t b = row / a.rows;
+    src[r] = static_cast<const T*>(a.t) + (b * a.t_rows + row - b * a.rows) * a.H;
+    acc[r] = 0.f;
+  }
+  const T* w = static_cast<const T*>(a.w);
+  for (int c = 8 * lane; c < a.H; c += 8 * 64) {
+    V8<T> wv, v[kBetaRows];
+    wv.raw = *reinterpret_cast<const u32x4*>(w + c);
+#pragma unroll
+    for (int r = 0; r < kBetaRows; ++r) v[r].raw = *reinterpret_cast<const u32x4*>(src[r] + c);
+#pragma unroll
+    for (int r = 0; r < kBetaRows; ++r)
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        acc[r] = fmaf(static_cast<float>(v[r].e[e]), static_cast<float>(wv.e[e]), acc[r]);
+  }
+  float mine = 0.f;
+#pragma unroll
+  for (int r = 0; r < kBetaRows; ++r) {
+#pragma unroll
+    for (int m = 1; m < 64; m <<= 1) acc[r] += __shfl_xor(acc[r], m, 64);
+    mine = lane == r ? acc[r] : mine;
+  }
+  if (lane < kBetaRows && r0 + lane < total) {
+    // the product rounded, then its sigmoid, as the two torch launches round
+    const float x = static_cast<float>(round_to<T>(mine));
+    static_cast<T*>(a.beta)[r0 + lane] = round_to<T>(1.0f / (1.0f + expf(-x)));
+  }
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
 template <typename T>
 hipError_t launch_pdbt(const TttProjBetaArgs& a, hipStream_t st) {
   const dim3 grid((a.H + kTile - 1) / kTile, (a.C + kTile - 1) / kTile, a.B * a.nupd);
-  hipLaunchKernelGGL(ttt_pd_beta_t_kernel<T>, grid, dim3(256), 0, st, a);
+  const bool vec = a.H % 8 == 0 && a.C % 8 == 0 && a.pd_stride % 8 == 0 && aligned16(a.pd) &&
+                   aligned16(a.pdt);
+  if (vec)
+    hipLaunchKernelGGL(ttt_pd_beta_t_vec_kernel<T>, grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(ttt_pd_beta_t_kernel<T>, grid, dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_scan(const TttScanArgs& a, hipStream_t st) {
   const dim3 grid((a.I + kTile - 1) / kTile, (a.H + kTile - 1) / kTile, 1);
-  hipLaunchKernelGGL(ttt_scan_kernel<T>, grid, dim3(256), 0, st, a);
+  const bool vec = a.H % 8 == 0 && a.I % 8 == 0 && aligned16(a.dw) && aligned16(a.w_cur) &&
+                   aligned16(a.steps_t) && aligned16(a.w_next);
+  if (vec)
+    hipLaunchKernelGGL(ttt_scan_vec_kernel<T>, grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(ttt_scan_kernel<T>, grid, dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_beta(const TttBetaArgs& a, hipStream_t st) {
+  const int64_t waves = ((int64_t)a.B * a.rows + kBetaRows - 1) / kBetaRows;
+  hipLaunchKernelGGL(ttt_beta_kernel<T>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
@@ -489,6 +692,10 @@ hipError_t launch_ttt_features(const TttFeatureArgs& a, Elem dtype, Elem w_dtype
 
 hipError_t launch_ttt_proj_beta_t(const TttProjBetaArgs& a, Elem dtype, hipStream_t stream) {
   return dtype == Elem::BF16 ? launch_pdbt<__bf16>(a, stream) : launch_pdbt<_Float16>(a, stream);
+}
+
+hipError_t launch_ttt_beta(const TttBetaArgs& a, Elem dtype, hipStream_t stream) {
+  return dtype == Elem::BF16 ? launch_beta<__bf16>(a, stream) : launch_beta<_Float16>(a, stream);
 }
 
 hipError_t launch_ttt_scan(const TttScanArgs& a, Elem dtype, hipStream_t stream) {

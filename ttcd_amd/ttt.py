@@ -179,6 +179,20 @@ def _gate_up(x: torch.Tensor, t: torch.Tensor, gate_up: torch.Tensor, n: int):
     return F.linear(x.view(rows, H), gate_up), F.linear(t.view(rows, H)[:n], gate_up)
 
 
+def _beta(t: torch.Tensor, b_proj: torch.Tensor, rows: int) -> torch.Tensor:
+    """(t @ b_proj).sigmoid() of the first `rows` tokens of every sequence of t
+    (B, L, H), each step rounded to the dtype (scanfuse.py:72-74): (B, rows)."""
+    B, L, H = t.shape
+    if (H % 8 or t.data_ptr() % 16 or b_proj.shape != (H,) or not b_proj.is_contiguous()
+            or b_proj.dtype != t.dtype or b_proj.device != t.device or b_proj.data_ptr() % 16):
+        return torch.matmul(t[:, :rows], b_proj).sigmoid().contiguous()
+    _check_gpu("ttt_mlp", t=t, b_proj=b_proj)
+    beta = torch.empty(B, rows, dtype=t.dtype, device=t.device)
+    _lib.check(_lib.lib().ttcd_ttt_beta_fwd(t.data_ptr(), L, b_proj.data_ptr(), beta.data_ptr(),
+                                            B, rows, H, _DT[t.dtype], _stream(t)))
+    return beta
+
+
 def proj_beta_t(pd: torch.Tensor, beta: torch.Tensor | None, B: int, nupd: int,
                 chunk: int) -> torch.Tensor:
     """pd (B*nupd*chunk, H) -> (B*nupd, H, chunk) = per chunk (pd * beta)^T,
@@ -351,13 +365,7 @@ def ttt_mlp(x: torch.Tensor, t: torch.Tensor, w: TttMlpWeights, *, chunk: int, l
     out = torch.empty(B, nchunk, C, H, dtype=dt, device=dev)
     beta = None
     if w.b_proj is not None:
-        # (t_padded @ b_proj).sigmoid(), bf16 (scanfuse.py:72-74)
-        # for the updating chunks (of a batch: for all rows, then cut). Rows as
-        # a matrix: with a leading dimension torch takes a GEMM of one column,
-        # 33 us instead of 15 for 20480 rows of 1024.
-        rows = t.view(B * L, H) if B > 1 else t[0, :upd]
-        beta = torch.matmul(rows, w.b_proj).sigmoid()
-        beta = beta.view(B, -1)[:, :upd].reshape(B, nchunk - 1, C).contiguous()
+        beta = _beta(t, w.b_proj, upd).view(B, nchunk - 1, C)
     W_upd_t = W_base.t()
     if w.ttt_proj is not None:
         W_upd_t = torch.matmul(W_base.t(), w.ttt_proj)  # (I, H), scanfuse.py:95-96
