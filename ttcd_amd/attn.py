@@ -42,10 +42,6 @@ def _rescale(exact_max: bool) -> float:
     return 0.0 if exact_max else LAZY_RESCALE_LOG2
 
 
-def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
-
-
 def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, fn: str):
     for name, t in (("q", q), ("k", k), ("v", v)):
         if not isinstance(t, torch.Tensor) or t.dim() != 4:
@@ -76,8 +72,11 @@ def _ready(t: torch.Tensor) -> torch.Tensor:
     """t itself when the C ABI takes it as is (unit head_dim stride, element
     strides multiples of 8, 16-byte aligned base), else a contiguous copy: a
     q / k / v view of one fused projection output needs no copy."""
-    if (t.stride(-1) == 1 and all(st % 8 == 0 for st in t.stride()[:-1])
-            and t.data_ptr() % 16 == 0):
+    st = t.stride()
+    if st[-1] == 1 and t.data_ptr() % 16 == 0:
+        for s in st[:-1]:
+            if s % 8:
+                return t.contiguous()
         return t
     return t.contiguous()
 
@@ -131,8 +130,8 @@ def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     q, k, v = _ready(q), _ready(k), _ready(v)
     # o_t and o_s are the two contiguous halves of one allocation, so the
     # epilogue can run one o_proj GEMM over both without a copy
-    both = torch.empty((2,) + tuple(q.shape), dtype=q.dtype, device=q.device)  # contiguous
-    ot, os_ = both[0], both[1]
+    both = q.new_empty((2,) + q.shape)
+    ot, os_ = both.select(0, 0), both.select(0, 1)
     lse_t = lse_s = None
     if return_lse:
         lse_t = torch.empty(B, H, T, device=q.device, dtype=torch.float32)
@@ -146,7 +145,7 @@ def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         _lse_ptr(lse_t), _lse_ptr(lse_s), B, T, k.shape[1], H, HK, D,
         _lib.strides4(q.stride()), _lib.strides4(k.stride()), _lib.strides4(v.stride()),
         _lib.strides4(ot.stride()), wt, ws, D ** -0.5, rescale, _DT[q.dtype],
-        _lse_ptr(work), nbytes, _stream(q.device)))
+        _lse_ptr(work), nbytes, _lib.stream(q)))
     if return_lse:
         return ot, os_, lse_t, lse_s
     return ot, os_
@@ -178,7 +177,7 @@ def band_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, band_lo: int, b
         B, T, Tk, H, HK, D,
         _lib.strides4(q.stride()), _lib.strides4(k.stride()), _lib.strides4(v.stride()),
         _lib.strides4(o.stride()), lo, hi, D ** -0.5, rescale, _DT[q.dtype],
-        _lse_ptr(work), nbytes, _stream(q.device)))
+        _lse_ptr(work), nbytes, _lib.stream(q)))
     return (o, lse) if return_lse else o
 
 
@@ -246,8 +245,8 @@ def fused_dual_window_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Ten
                                           "fused_dual_window_attn_varlen")
     wt = -1 if (window_teacher is None or window_teacher < 0) else window_teacher
     q, k, v = _ready(q), _ready(k), _ready(v)
-    both = torch.empty((2,) + tuple(q.shape), dtype=q.dtype, device=q.device)
-    ot, os_ = both[0], both[1]
+    both = q.new_empty((2,) + q.shape)
+    ot, os_ = both.select(0, 0), both.select(0, 1)
     lse_t = lse_s = None
     if return_lse:
         lse_t = torch.empty(H, total, device=q.device, dtype=torch.float32)
@@ -261,7 +260,7 @@ def fused_dual_window_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Ten
         H, HK, D, _lib.strides3(q.stride()), _lib.strides3(k.stride()),
         _lib.strides3(v.stride()), _lib.strides3(ot.stride()), int(min(wt, 2**31 - 1)),
         int(min(window_student, 2**31 - 1)), D ** -0.5, _rescale(exact_max), _DT[q.dtype],
-        _stream(q.device)))
+        _lib.stream(q)))
     if return_lse:
         return ot, os_, lse_t, lse_s
     return ot, os_
@@ -290,7 +289,7 @@ def band_attn_varlen(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         cu_seqlens.data_ptr(), nseq, int(max_seqlen), total, H, HK, D,
         _lib.strides3(q.stride()), _lib.strides3(k.stride()), _lib.strides3(v.stride()),
         _lib.strides3(o.stride()), int(min(band_lo, 2**31 - 1)), int(min(band_hi, 2**31 - 1)),
-        D ** -0.5, _rescale(exact_max), _DT[q.dtype], _stream(q.device)))
+        D ** -0.5, _rescale(exact_max), _DT[q.dtype], _lib.stream(q)))
     return (o, lse) if return_lse else o
 
 
@@ -314,7 +313,7 @@ def lse_merge(o_s: torch.Tensor, lse_s: torch.Tensor, o_f: torch.Tensor, lse_f: 
     _lib.check(L.ttcd_lse_merge_fwd(
         o_s.data_ptr(), lse_s.data_ptr(), o_f.data_ptr(), lse_f.data_ptr(), o_t.data_ptr(),
         B, T, H, D, int(row_start), _lib.strides4(o_s.stride()), _DT[o_s.dtype],
-        _stream(o_s.device)))
+        _lib.stream(o_s)))
     return o_t
 
 
@@ -337,8 +336,8 @@ def lse_dual_window_attn(q, k, v, window_teacher: int, window_student: int, *,
     B, Tq, H, HK, D = _check_qkv(q, k, v, "lse_dual_window_attn")
     q, k, v = _ready(q), _ready(k), _ready(v)
     # o_t and o_s as the halves of one allocation (see fused_dual_window_attn)
-    both = torch.empty((2,) + tuple(q.shape), dtype=q.dtype, device=q.device)
-    ot, os_ = both[0], both[1]
+    both = q.new_empty((2,) + q.shape)
+    ot, os_ = both.select(0, 0), both.select(0, 1)
     L = _lib.lib()
     WS_ = int(min(WS, 2**31 - 1))
     nbytes = L.ttcd_lse_dual_window_attn_workspace_bytes(B, Tq, Tk, H, D, WS_)
@@ -347,7 +346,7 @@ def lse_dual_window_attn(q, k, v, window_teacher: int, window_student: int, *,
         q.data_ptr(), k.data_ptr(), v.data_ptr(), ot.data_ptr(), os_.data_ptr(), B, Tq, Tk, H,
         HK, D, _lib.strides4(q.stride()), _lib.strides4(k.stride()), _lib.strides4(v.stride()),
         _lib.strides4(ot.stride()), int(min(WT, 2**31 - 1)), WS_, D ** -0.5,
-        _rescale(exact_max), _DT[q.dtype], ws.data_ptr(), int(nbytes), _stream(q.device)))
+        _rescale(exact_max), _DT[q.dtype], ws.data_ptr(), int(nbytes), _lib.stream(q)))
     return ot, os_
 
 

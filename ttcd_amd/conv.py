@@ -43,7 +43,7 @@ def causal_dwconv_x(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     L = _lib.lib()
     _lib.check(L.ttcd_causal_dwconv_chunked_fwd(
         x.data_ptr(), w.data_ptr(), y.data_ptr(), N, C, D, K, _DT[x.dtype], _DT[w.dtype],
-        torch.cuda.current_stream(x.device).cuda_stream))
+        _lib.stream(x)))
     return y
 
 

@@ -64,8 +64,8 @@ def dual_residual_rmsnorm(attn_t: torch.Tensor, attn_s: torch.Tensor, residual: 
     w = weight.contiguous()
     # hidden_states and student_output are the two halves of one allocation, so
     # the TTT MLP can run its gate/up GEMM over both without a copy
-    ys = torch.empty((2,) + tuple(res.shape), dtype=res.dtype, device=res.device)
-    y_t, y_s = ys[0], ys[1]
+    ys = res.new_empty((2,) + res.shape)
+    y_t, y_s = ys.select(0, 0), ys.select(0, 1)
     res_out = torch.empty_like(res)
     rows = res.numel() // H if H > 0 else 0
     if rows == 0:  # nothing to launch (an empty tensor's data pointer may be null)
@@ -73,7 +73,7 @@ def dual_residual_rmsnorm(attn_t: torch.Tensor, attn_s: torch.Tensor, residual: 
     _lib.check(_lib.lib().ttcd_dual_residual_rmsnorm_fwd(
         a_t.data_ptr(), a_s.data_ptr(), res.data_ptr(), w.data_ptr(), _DT[w.dtype], float(eps),
         y_t.data_ptr(), res_out.data_ptr(), y_s.data_ptr(), rows, H, _DT[res.dtype],
-        torch.cuda.current_stream(res.device).cuda_stream))
+        _lib.stream(res)))
     return y_t, res_out, y_s
 
 
@@ -111,7 +111,7 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
             x.data_ptr(), res.data_ptr() if res is not None else None, w.data_ptr(),
             _DT[w.dtype], float(eps), y.data_ptr(),
             res_out.data_ptr() if res_out is not None else None, rows, H, _DT[x.dtype],
-            torch.cuda.current_stream(x.device).cuda_stream))
+            _lib.stream(x)))
     return y if res is None else (y, res_out)
 
 
@@ -138,7 +138,7 @@ def add_rmsnorm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor, e
     if rows > 0:
         _lib.check(_lib.lib().ttcd_add_rmsnorm_fwd(
             x.data_ptr(), res.data_ptr(), w.data_ptr(), _DT[w.dtype], float(eps), y.data_ptr(),
-            h.data_ptr(), rows, H, _DT[x.dtype], torch.cuda.current_stream(x.device).cuda_stream))
+            h.data_ptr(), rows, H, _DT[x.dtype], _lib.stream(x)))
     return y, h
 
 

@@ -298,10 +298,8 @@ class IPTTCDv9Prefill:
         c, w = self.cfg, self.w
         B, T, _ = x.shape
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
-        qkv = F.linear(x, self.qkv_w[i])
-        q = qkv[..., :Hq * D].view(B, T, Hq, D)
-        k = qkv[..., Hq * D:(Hq + Hkv) * D].view(B, T, Hkv, D)
-        v = qkv[..., (Hq + Hkv) * D:].view(B, T, Hkv, D)
+        qkv = F.linear(x, self.qkv_w[i]).view(B, T, Hq + 2 * Hkv, D)
+        q, k, v = qkv.split((Hq, Hkv, Hkv), 2)
         p = f"model.layers.{i}.attn."
         cos, sin = ctx.tables if ctx.tables is not None else self.tables(ctx.offset + T)
         qw = w.get(p + "q_norm.weight") if c["qk_norm"] else None

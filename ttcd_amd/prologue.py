@@ -35,10 +35,6 @@ _DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16,
        torch.float32: _lib.DTYPE_F32}
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
-
-
 def rope_inv_freq(dim: int, base: float, device=None) -> torch.Tensor:
     """1 / base ** (arange(0, dim, 2) / dim) in fp32, as
     RotaryEmbedding._compute_inv_freq (fla/modules/rotary.py:418-425, no YaRN)."""
@@ -61,7 +57,7 @@ def rope_tables(inv_freq: torch.Tensor, rows: int,
     cos = torch.empty(rows, half, dtype=dtype, device=inv.device)
     sin = torch.empty(rows, half, dtype=dtype, device=inv.device)
     _lib.check(_lib.lib().ttcd_rope_table_fwd(cos.data_ptr(), sin.data_ptr(), inv.data_ptr(),
-                                              int(rows), half, _DT[dtype], _stream(inv)))
+                                              int(rows), half, _DT[dtype], _lib.stream(inv)))
     return cos, sin
 
 
@@ -110,8 +106,8 @@ def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, q_norm_weight: torch.Tensor |
             raise ValueError("qk_norm_rope: norm weights must share one of bf16, f16, f32")
         wq, wk = q_norm_weight.contiguous(), k_norm_weight.contiguous()
         w_code = _DT[wq.dtype]
-    q_out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    k_out = torch.empty(k.shape, dtype=k.dtype, device=k.device)
+    q_out = q.new_empty(q.shape)
+    k_out = k.new_empty(k.shape)
     cos_c, sin_c = cos.contiguous(), sin.contiguous()
     _lib.check(_lib.lib().ttcd_qk_norm_rope_fwd(
         q.data_ptr(), k.data_ptr(), q_out.data_ptr(), k_out.data_ptr(),
@@ -119,7 +115,7 @@ def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, q_norm_weight: torch.Tensor |
         w_code, float(eps), cos_c.data_ptr(), sin_c.data_ptr(), cos_c.shape[0],
         B, T, Hq, k.shape[2], D, _lib.strides4(q.stride()), _lib.strides4(k.stride()),
         _lib.strides4(q_out.stride()), _lib.strides4(k_out.stride()), int(seqlen_offset),
-        _DT[q.dtype], _stream(q)))
+        _DT[q.dtype], _lib.stream(q)))
     return q_out, k_out
 
 

@@ -27,10 +27,6 @@ _DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16,
        torch.float32: _lib.DTYPE_F32}
 
 
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
-
-
 def _check_gpu(fn: str, **tensors):
     for name, t in tensors.items():
         if t is None:
@@ -49,13 +45,13 @@ def _row_stride(t: torch.Tensor, fn: str, name: str) -> int:
         raise ValueError(f"{fn}: {name} must have a contiguous last dim")
     if t.dim() == 1 or t.is_contiguous():
         return t.shape[-1]
-    st = t.stride(-2)
-    expect = st
-    for d in range(t.dim() - 2, -1, -1):
-        if t.shape[d] != 1 and t.stride(d) != expect:
+    shape, strides = t.shape, t.stride()
+    expect = strides[-2]
+    for n, st in zip(shape[-2::-1], strides[-2::-1]):
+        if n != 1 and st != expect:
             raise ValueError(f"{fn}: {name} rows must be evenly strided")
-        expect *= t.shape[d]
-    return st
+        expect *= n
+    return strides[-2]
 
 
 def swiglu(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
@@ -73,7 +69,7 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None
     if rows:
         _lib.check(_lib.lib().ttcd_swiglu_fwd(
             gate.data_ptr(), up.data_ptr(), out.data_ptr(), rows, cols, g_st, u_st,
-            _row_stride(out, "swiglu", "out"), _DT[gate.dtype], _stream(gate)))
+            _row_stride(out, "swiglu", "out"), _DT[gate.dtype], _lib.stream(gate)))
     return out
 
 
@@ -133,7 +129,7 @@ def ttt_features(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tensor | 
         ws[0].data_ptr() if ws[0] is not None else None,
         ws[1].data_ptr() if ws[1] is not None else None, _DT[wdt], K, z.data_ptr(),
         z_hat.data_ptr(), diff.data_ptr() if nchunk > 1 else None, B, nchunk, chunk, I,
-        _DT[dt], _stream(gu_t)))
+        _DT[dt], _lib.stream(gu_t)))
     return z, z_hat, diff
 
 
@@ -162,7 +158,7 @@ def _features_tokens(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tenso
         gu_t.data_ptr(), tokens, gu_s.data_ptr(), tokens, gu_t.stride(0),
         ws[0].data_ptr() if ws[0] is not None else None,
         ws[1].data_ptr() if ws[1] is not None else None, _DT[wdt], K, z.data_ptr(),
-        z_hat.data_ptr(), diff.data_ptr(), B, tokens, chunk, I, _DT[dt], _stream(gu_t)))
+        z_hat.data_ptr(), diff.data_ptr(), B, tokens, chunk, I, _DT[dt], _lib.stream(gu_t)))
     return z, z_hat, diff
 
 
@@ -189,7 +185,7 @@ def _beta(t: torch.Tensor, b_proj: torch.Tensor, rows: int) -> torch.Tensor:
     _check_gpu("ttt_mlp", t=t, b_proj=b_proj)
     beta = torch.empty(B, rows, dtype=t.dtype, device=t.device)
     _lib.check(_lib.lib().ttcd_ttt_beta_fwd(t.data_ptr(), L, b_proj.data_ptr(), beta.data_ptr(),
-                                            B, rows, H, _DT[t.dtype], _stream(t)))
+                                            B, rows, H, _DT[t.dtype], _lib.stream(t)))
     return beta
 
 
@@ -211,7 +207,7 @@ def proj_beta_t(pd: torch.Tensor, beta: torch.Tensor | None, B: int, nupd: int,
     out = torch.empty(B * nupd, H, chunk, dtype=pd.dtype, device=pd.device)
     _lib.check(_lib.lib().ttcd_ttt_proj_beta_t_fwd(
         pd.data_ptr(), pd.stride(0), beta.data_ptr() if beta is not None else None, bsb,
-        out.data_ptr(), B, nupd, chunk, H, _DT[pd.dtype], _stream(pd)))
+        out.data_ptr(), B, nupd, chunk, H, _DT[pd.dtype], _lib.stream(pd)))
     return out
 
 
@@ -237,7 +233,7 @@ def scan_steps(dw: torch.Tensor | None, w_cur: torch.Tensor, lr: float, nsteps: 
     _lib.check(_lib.lib().ttcd_ttt_scan_fwd(
         dw.data_ptr() if dw is not None else None, w_cur.data_ptr(), lr_q, steps.data_ptr(),
         w_next.data_ptr() if w_next is not None else None, nupd, nsteps, H, I, _DT[dt],
-        _stream(w_cur)))
+        _lib.stream(w_cur)))
     return steps, w_next
 
 
