@@ -1,0 +1,67 @@
+"""Projections of few rows (ttcd_amd.linear): the kernel against 64 bits at the
+edges of its tiles, its SwiGLU form against its own product, and what is left
+to torch.
+
+Bound: the fp32 sum of K products is off by at most K 2^-24 of the sum of their
+magnitudes, and the result is rounded once, u |y|."""
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from ttcd_amd import _lib, linear as L, ttt
+
+
+def _xw(shape, N, K, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(*shape, K, generator=g).to(dtype).cuda()
+    return x, (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype).cuda()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,N,K,dtype", [
+    ((1,), 16, 32, torch.bfloat16), ((1, 16), 24, 96, torch.float16), ((2, 8), 1, 1024, torch.bfloat16),
+    ((17,), 1000, 960, torch.bfloat16), ((3, 11), 4096, 1024, torch.bfloat16),
+    ((1, 64), 1024, 3072, torch.float16), ((48,), 8200, 256, torch.bfloat16),
+    ((64,), 6144, 1056, torch.bfloat16)])
+@torch.inference_mode()
+def test_few_rows_match_64_bits(gpu, shape, N, K, dtype):
+    x, w = _xw(shape, N, K, dtype, N + K)
+    got = L.linear(x, w)
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    want = x.double() @ w.double().T
+    limit = u * want.abs() + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert got.shape == shape + (N,) and got.dtype == dtype
+    assert ((got.double() - want).abs() <= limit).all()
+    if N % 2 == 0 and N % 16 == 0:
+        z = L.swiglu_linear(x, w)
+        assert torch.equal(z, ttt.swiglu(got[..., :N // 2], got[..., N // 2:]))
+
+
+@pytest.mark.gpu
+def test_what_is_left_to_torch(gpu):
+    x, w = _xw((65,), 64, 64, torch.bfloat16, 1)
+    assert L._rows_for_kernel(x[:64], w) == 64
+    for a, b in ((x, w), (x[:8, :48], w[:, :48]), (x[:8].float(), w.float()), (x[:8].t(), w[:, :8]),
+                 (x[:8], w[::2]), (x.flatten()[1:65].view(1, 64), w), (x[:0], w)):
+        assert L._rows_for_kernel(a, b) == 0
+        assert torch.equal(L.linear(a, b), F.linear(a, b))
+        assert L.swiglu_linear(a, b) is None
+    wg = w.clone().requires_grad_()
+    y = L.linear(x[:8], wg)
+    assert y.requires_grad and L._rows_for_kernel(x[:8], wg) == 0
+    with torch.no_grad():
+        assert L._rows_for_kernel(x[:8], wg) == 8
+    with torch.autograd.forward_ad.dual_level():
+        assert L._rows_for_kernel(x[:8], w) == 0
+
+
+def test_cpu_tensors_and_bad_arguments():
+    x, w = torch.randn(4, 64), torch.randn(8, 64)
+    assert torch.equal(L.linear(x, w), F.linear(x, w))
+    C, P = _lib.lib(), 0x10000
+    call = lambda x=P, st=64, w=P, M=4, N=8, K=64, dt=0: C.ttcd_linear_rows_fwd(  # noqa: E731
+        x, st, w, P, M, N, K, 0, dt, None)
+    assert call(x=None) == call(M=0) == call(st=32) == _lib.TTCD_ERR_INVALID_ARGUMENT
+    assert call(K=48) == call(dt=2) == call(w=P + 2) == call(st=65) == _lib.TTCD_ERR_UNSUPPORTED

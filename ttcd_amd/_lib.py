@@ -52,6 +52,7 @@ EXPORTS = (
     "ttcd_rmsnorm_fwd",
     "ttcd_add_rmsnorm_fwd",
     "ttcd_swiglu_fwd",
+    "ttcd_linear_rows_fwd",
     "ttcd_ttt_features_fwd",
     "ttcd_ttt_features_tokens_fwd",
     "ttcd_ttt_proj_beta_t_fwd",
@@ -144,6 +145,7 @@ _SIGS = {
     "ttcd_add_rmsnorm_fwd": (_i32, [
         _vp, _vp, _vp, _i32, ctypes.c_float, _vp, _vp, _i64, _i32, _i32, _vp]),
     "ttcd_swiglu_fwd": (_i32, [_vp, _vp, _vp, _i64, _i32, _i64, _i64, _i64, _i32, _vp]),
+    "ttcd_linear_rows_fwd": (_i32, [_vp, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp]),
     "ttcd_ttt_features_fwd": (_i32, [
         _vp, _vp, _i64, _vp, _vp, _i32, _i32, _vp, _vp, _vp,
         _i32, _i32, _i32, _i32, _i32, _vp]),

@@ -987,6 +987,23 @@ ttcd_status ttcd_swiglu_fwd(const void* gate, const void* up, void* out, int64_t
                   "swiglu launch");
 }
 
+ttcd_status ttcd_linear_rows_fwd(const void* x, int64_t x_stride, const void* w, void* y, int M,
+                                 int N, int K, int swiglu, ttcd_dtype dtype, void* stream) {
+  if (!x || !w || !y) return fail(TTCD_ERR_INVALID_ARGUMENT, "null pointer argument");
+  if (M < 1 || N < 1 || K < 1 || x_stride < K)
+    return fail(TTCD_ERR_INVALID_ARGUMENT, "need M, N, K >= 1 and x_stride >= K");
+  if (dtype != TTCD_DTYPE_BF16 && dtype != TTCD_DTYPE_F16)
+    return fail(TTCD_ERR_UNSUPPORTED, "dtype must be bf16 or f16");
+  if (K % 32 != 0 || x_stride % 8 != 0)
+    return fail(TTCD_ERR_UNSUPPORTED, "K must be a multiple of 32 and x_stride of 8");
+  if (!aligned16(x) || !aligned16(w))
+    return fail(TTCD_ERR_UNSUPPORTED, "x and w must be 16-byte aligned");
+  if ((M + 15) / 16 > 65535) return fail(TTCD_ERR_UNSUPPORTED, "too many rows (grid y)");
+  const ttcd::LinearArgs a{x, x_stride, w, y, M, N, K, swiglu != 0};
+  return from_hip(ttcd::launch_linear_rows(a, elem(dtype), static_cast<hipStream_t>(stream)),
+                  "linear launch");
+}
+
 // Both forms of the feature pass.
 static ttcd_status ttt_features(const ttcd::TttFeatureArgs& a, ttcd_dtype w_dtype,
                                 ttcd_dtype dtype, void* stream) {

@@ -146,6 +146,18 @@ hipError_t launch_ttt_proj_beta_t(const TttProjBetaArgs& a, Elem dtype, hipStrea
 hipError_t launch_ttt_beta(const TttBetaArgs& a, Elem dtype, hipStream_t stream);
 hipError_t launch_ttt_scan(const TttScanArgs& a, Elem dtype, hipStream_t stream);
 
+// y = x w^T for few rows of x (linear.hip): x (M, K) with row stride x_st, w
+// (N, K) and y (M, N) contiguous; glu: w (2N, K) is gate | up and y their SwiGLU.
+struct LinearArgs {
+  const void* x;
+  int64_t x_st;
+  const void* w;
+  void* y;
+  int M, N, K;
+  bool glu;
+};
+hipError_t launch_linear_rows(const LinearArgs& a, Elem dtype, hipStream_t stream);
+
 hipError_t launch_dwconv(const void* x, const void* w, void* y, int64_t N, int C,
                          int D, int K, Elem xt, Elem wt, hipStream_t stream);
 

@@ -62,6 +62,7 @@
 #include <stdint.h>
 
 #include "internal.h"
+#include "silu.h"
 
 namespace ttcd {
 namespace {
@@ -73,32 +74,6 @@ union V8 {
   u32x4 raw;
   T e[8];
 };
-
-// Rounded to T as a separate step from the fp32 result (no fused
-// multiply-and-convert), as the reference stores an fp32 value.
-template <typename T>
-__device__ __forceinline__ T round_to(float v) {
-  asm volatile("" : "+v"(v));
-  return static_cast<T>(v);
-}
-
-// (g * s) * u with s = 1 / (1 + exp(-g)) in fp32. exp(-g) = 2^hi (1 + lo ln 2)
-// with hi + lo = -g log2(e) to ~48 bits, and one Newton step on the
-// reciprocal: 13 VALU operations beside the two quarter-rate ones, where expf
-// and the division take 25 and more. Past |g| = 120 the exponential is 0 or
-// infinite either way; an infinite denominator keeps its reciprocal 0.
-__device__ __forceinline__ float silu_mul(float g, float u) {
-  constexpr float kLog2e = 1.44269504088896341f;
-  constexpr float kLog2eLo = (float)(1.44269504088896340736 - (double)kLog2e);
-  constexpr float kLn2 = 0.693147180559945309f;
-  const float n = __builtin_amdgcn_fmed3f(-g, -120.f, 120.f);
-  const float hi = n * kLog2e;
-  const float lo = fmaf(n, kLog2eLo, fmaf(n, kLog2e, -hi));
-  const float d = 1.0f + __builtin_amdgcn_exp2f(hi) * fmaf(lo, kLn2, 1.0f);
-  const float r = __builtin_amdgcn_rcpf(d);
-  const float s = d < INFINITY ? fmaf(fmaf(-d, r, 1.0f), r, r) : r;
-  return (g * s) * u;
-}
 
 template <typename T>
 __global__ __launch_bounds__(256) void swiglu_kernel(const T* __restrict__ gate,
