@@ -24,7 +24,12 @@ def _xw(shape, N, K, dtype, seed):
     ((1,), 16, 32, torch.bfloat16), ((1, 16), 24, 96, torch.float16), ((2, 8), 1, 1024, torch.bfloat16),
     ((17,), 1000, 960, torch.bfloat16), ((3, 11), 4096, 1024, torch.bfloat16),
     ((1, 64), 1024, 3072, torch.float16), ((48,), 8200, 256, torch.bfloat16),
-    ((64,), 6144, 1056, torch.bfloat16)])
+    ((64,), 6144, 1056, torch.bfloat16),
+    # 64 x 64 tiles: one step, an odd number of steps for two groups, both sides
+    # of 256 tiles, ragged rows and columns; K that tiles do not take
+    ((65,), 64, 64, torch.bfloat16), ((2, 50), 1000, 576, torch.float16), ((129,), 66, 448, torch.bfloat16),
+    ((512,), 1024, 3072, torch.bfloat16), ((3, 100), 6144, 1024, torch.bfloat16),
+    ((65,), 16384, 960, torch.float16), ((511,), 3, 512, torch.bfloat16), ((70,), 96, 96, torch.bfloat16)])
 @torch.inference_mode()
 def test_few_rows_match_64_bits(gpu, shape, N, K, dtype):
     x, w = _xw(shape, N, K, dtype, N + K)
@@ -41,9 +46,9 @@ def test_few_rows_match_64_bits(gpu, shape, N, K, dtype):
 
 @pytest.mark.gpu
 def test_what_is_left_to_torch(gpu):
-    x, w = _xw((65,), 64, 64, torch.bfloat16, 1)
-    assert L._rows_for_kernel(x[:64], w) == 64
-    for a, b in ((x, w), (x[:8, :48], w[:, :48]), (x[:8].float(), w.float()), (x[:8].t(), w[:, :8]),
+    x, w = _xw((513,), 64, 64, torch.bfloat16, 1)
+    assert L._rows_for_kernel(x[:512], w) == 512
+    for a, b in ((x, w), (x[:8, :48], w[:, :48]), (x[:8].float(), w.float()), (x[:64].t(), w),
                  (x[:8], w[::2]), (x.flatten()[1:65].view(1, 64), w), (x[:0], w)):
         assert L._rows_for_kernel(a, b) == 0
         assert torch.equal(L.linear(a, b), F.linear(a, b))

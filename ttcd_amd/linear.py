@@ -1,13 +1,13 @@
 """Projections without a bias: y = x @ w.T, and the SwiGLU of a stacked gate|up
 projection (host side of linear.hip).
 
-Up to MAX_ROWS rows of x take the HIP kernel, everything else torch's GEMM
-(hipBLASLt). The line is where the kernel stops being the faster on the GPU
-(us, kernel / GEMM, weights not in cache): 4096 x 1024 16 rows 4.7 / 6.0, 64 rows
-7.7 / 8.8, 128 rows 12.7 / 9.3; 1024 x 3072 16 rows 8.8 / 9.3, 64 rows 8.5 /
-9.9, 128 rows 11.8 / 8.2. Below it the call counts too: 4 us of host time
-instead of 17. Wide outputs (a vocabulary's logits) stay with the GEMM, which
-streams them faster from 8 rows on (151936 x 1024: 78 / 61 us).
+Up to MAX_ROWS rows of x take the HIP kernels, everything else torch's GEMM
+(hipBLASLt). Up to 64 rows the kernel is the faster on the GPU, up to 512 they
+are about even (linear.hip has the times), and a call of it takes 7 us of host
+time instead of 17, which is what a short prompt's layer is made of. Past 512
+rows the GEMM runs longer than its call and is the faster of the two (4096 x
+1024, 1000 rows: 17 / 13 us). Wide outputs (a vocabulary's logits) stay with
+the GEMM, which streams them faster from 8 rows on (151936 x 1024: 78 / 61 us).
 """
 from __future__ import annotations
 
@@ -19,7 +19,7 @@ from . import _lib
 
 _DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}
 
-MAX_ROWS = 64
+MAX_ROWS = 512
 MAX_COLS = 16384
 
 
