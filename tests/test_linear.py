@@ -24,7 +24,7 @@ def _xw(shape, N, K, dtype, seed):
     ((1,), 16, 32, torch.bfloat16), ((1, 16), 24, 96, torch.float16), ((2, 8), 1, 1024, torch.bfloat16),
     ((17,), 1000, 960, torch.bfloat16), ((3, 11), 4096, 1024, torch.bfloat16),
     ((1, 64), 1024, 3072, torch.float16), ((48,), 8200, 256, torch.bfloat16),
-    ((64,), 6144, 1056, torch.bfloat16),
+    ((64,), 6144, 1056, torch.bfloat16), ((40,), 8192, 128, torch.bfloat16),
     # 64 x 64 tiles: one step, an odd number of steps for two groups, both sides
     # of 256 tiles, ragged rows and columns; K that tiles do not take
     ((65,), 64, 64, torch.bfloat16), ((2, 50), 1000, 576, torch.float16), ((129,), 66, 448, torch.bfloat16),

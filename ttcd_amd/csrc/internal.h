@@ -1,5 +1,6 @@
 // internal.h - launcher interface between the C ABI (api.hip) and the
-// gfx950 kernels (attn.hip, conv.hip, merge.hip, prologue.hip, epilogue.hip).
+// gfx950 kernels (attn.hip, conv.hip, merge.hip, prologue.hip, epilogue.hip,
+// ttt.hip, linear.hip).
 // Not part of the ABI.
 #pragma once
 
