@@ -112,3 +112,38 @@ def test_split_call_under_graph_capture(gpu):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,HK,D,dtype", [
+    (16, 8, 128, torch.bfloat16), (4, 4, 128, torch.float16), (15, 5, 64, torch.bfloat16),
+    (4, 2, 64, torch.float16)])
+@pytest.mark.parametrize("Tq,Tk,ws,near,far", [
+    (40, 8231, 1000, 5.0, 55.0), (40, 8231, 1000, 5.0, 95.0), (40, 8231, 1000, 5.0, 105.0),
+    (40, 8231, 1000, 5.0, 205.0), (40, 8231, 4096, 150.0, -50.0),
+    # rows without a far key among rows with some, every score far below zero
+    (200, 9000, 8900, -150.0, -150.0)])
+@torch.inference_mode()
+def test_near_and_far_scores_far_apart(gpu, Tq, Tk, ws, near, far, H, HK, D, dtype):
+    """Scores offset by `near` nats within the student window and by `far` beyond it, up to
+    200 apart, past what exp spans in fp32: the student is its own window's
+    softmax however large the far scores are. An LSE of size |L| is a product and
+    sums in fp32: eight units of L in either call."""
+    q, k, v = make_qkv(batch=1, seqlen=Tk, heads=H, kv_heads=HK, head_dim=D, dtype=dtype,
+                       seed=Tk + ws)
+    q = q[:, Tk - Tq:].clone()
+    q[..., 0] = 16.0
+    reach = Tk - Tq - ws + 1 if near != far else 0  # keys no row's student window holds
+    k[..., 0] = near / (16.0 * D ** -0.5)
+    k[:, :reach, :, 0] = far / (16.0 * D ** -0.5)
+    assert _bytes(1, Tq, Tk, H, HK, D, 0, ws, Tk) > 0
+    got = fused_dual_window_attn(q, k, v, -1, ws, return_lse=True)
+    want = _whole(q, k, v, 0, ws, Tk, True)
+    assert all(torch.isfinite(x).all() for x in got)
+    if near != far:
+        gap = want[2] - want[3]
+        assert (gap - max(far - near, 0.0)).abs().max() < 12.0  # the keys' own spread
+    for name, g, w, W in (("teacher", got[0], want[0], Tk), ("student", got[1], want[1], ws)):
+        _close(g, w, 1.02 * window_attn(q, k, v.abs(), W).float(), dtype, name)
+    for g, w in ((got[2], want[2]), (got[3], want[3])):
+        assert ((g - w).abs() <= 1e-5 + 2.0 ** -21 * w.abs()).all()

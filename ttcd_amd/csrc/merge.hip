@@ -13,8 +13,11 @@
 //
 // attn_combine_kernel is the same identity for an attention call split over
 // keys into any number of fp32 parts (attn.hip, PART): weights exp(lse_p - m)
-// with m the row's largest LSE, one division and one rounding at the end; the
-// near parts' running sums give the student's output on the way.
+// with m the row's largest LSE, one division and one rounding at the end. The
+// near parts are added first, under the largest LSE of their own: the student's
+// output is their sum alone, and far keys may outscore the near ones by more
+// than exp can span in fp32 (88). Their sums are then rescaled to the whole
+// row's reference, as an online softmax does.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -108,9 +111,14 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs a) {
   const float* src = a.part + row * a.D + dg * 8;
   const int64_t off = b * a.sb + t * a.st + h * a.sh + dg * 8;
 
-  float m = -INFINITY;
-  for (int p = 0; p < a.parts; ++p) m = fmaxf(m, a.part_lse[p * rows + li]);
-  const float ref = m == -INFINITY ? 0.f : m;
+  auto largest = [&](int p0, int p1) {
+    float m = -INFINITY;
+    for (int p = p0; p < p1; ++p) m = fmaxf(m, a.part_lse[p * rows + li]);
+    return m;
+  };
+  const bool near = a.o_near != nullptr;
+  float m = largest(0, near ? a.near_parts : a.parts);
+  float ref = m == -INFINITY ? 0.f : m;  // no key in any of them: every weight is 0
   float acc[8], sum = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
@@ -123,7 +131,17 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs a) {
     if (lse != nullptr && dg == 0) lse[li] = sum > 0.f ? ref + logf(sum) : -INFINITY;
   };
   for (int p = 0; p < a.parts; ++p) {
-    if (p == a.near_parts && a.o_near != nullptr) emit(a.o_near, a.lse_near);
+    if (p == a.near_parts && near) {
+      emit(a.o_near, a.lse_near);
+      const float far = largest(p, a.parts);
+      if (far > m) {  // the factor is 0 when no near part had a key (m = -inf)
+        const float scale = expf(m - far);
+        sum *= scale;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[e] *= scale;
+        m = ref = far;
+      }
+    }
     const float w = expf(a.part_lse[p * rows + li] - ref);
     const f32x4* v = reinterpret_cast<const f32x4*>(src + p * rows * a.D);
     const f32x4 lo = __builtin_nontemporal_load(v), hi = __builtin_nontemporal_load(v + 1);
@@ -134,7 +152,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs a) {
       acc[4 + e] = fmaf(hi[e], w, acc[4 + e]);
     }
   }
-  if (a.near_parts == a.parts && a.o_near != nullptr) emit(a.o_near, a.lse_near);
+  if (a.near_parts == a.parts && near) emit(a.o_near, a.lse_near);
   emit(a.o, a.lse);
 }
 
