@@ -121,3 +121,25 @@ def test_scan_on_whole_groups(gpu, nupd, nsteps, H, I, want_next):
     for s_ in range(nsteps):
         assert torch.equal(steps[s_], ws[s_].t()), s_
     assert nxt is None if not want_next else torch.equal(nxt, ws[nupd])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("u", [1.0, -0.375, 250.0, 2.0 ** -10])
+@torch.inference_mode()
+def test_swiglu_of_every_gate(gpu, dtype, u):
+    """Every bit pattern of the gate, where 1 + exp(-g) leaves fp32 and next to it
+    included, against (g * (1 / (1 + exp(-g)))) * u in fp32 on the CPU: a few
+    units of fp32 (2^-20) and one rounding to the dtype (its unit, or half its
+    smallest subnormal); infinities and NaN where the formula has them."""
+    g = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(dtype)
+    got = ttt.swiglu(g.cuda().view(64, 1024), torch.full((64, 1024), u, dtype=dtype, device=gpu))
+    got = got.cpu().view(-1)
+    gf = g.float()
+    want = gf * (1.0 / (1.0 + torch.exp(-gf))) * u
+    unit, least = (2.0 ** -8, 2.0 ** -134) if dtype == torch.bfloat16 else (2.0 ** -11, 2.0 ** -25)
+    rounded = want.to(dtype)
+    assert torch.equal(got.isnan(), want.isnan())
+    finite = rounded.isfinite()
+    assert torch.equal(got[~finite & ~want.isnan()], rounded[~finite & ~want.isnan()])
+    w = want[finite].double()
+    assert ((got[finite].double() - w).abs() <= (unit + 2.0 ** -20) * w.abs() + least).all()
