@@ -70,3 +70,24 @@ def test_cpu_tensors_and_bad_arguments():
         x, st, w, P, M, N, K, 0, dt, None)
     assert call(x=None) == call(M=0) == call(st=32) == _lib.TTCD_ERR_INVALID_ARGUMENT
     assert call(K=48) == call(dt=2) == call(w=P + 2) == call(st=65) == _lib.TTCD_ERR_UNSUPPORTED
+
+
+def test_the_kernel_is_chosen_by_shape():
+    """Both sides of the lines that the kernel's and the GEMM's times draw (_pays)."""
+    kernel = [(1, 4096, 11008, 0), (16, 6144, 1024, 0), (64, 1024, 3072, 0), (64, 4096, 1024, 0),
+              (64, 6144, 1024, 1), (65, 1024, 2048, 0), (512, 4096, 1024, 0), (384, 6144, 1024, 0),
+              (512, 6144, 1024, 1), (256, 4096, 4096, 0), (300, 1024, 3072, 0)]
+    gemm = [(16, 16384, 4096, 0), (17, 4096, 11008, 0), (64, 6144, 1024, 0), (64, 4096, 4096, 0),
+            (65, 1024, 3072, 0), (256, 1024, 3072, 0), (128, 960, 2560, 0), (2, 384, 6016, 1),
+            (512, 6144, 1024, 0), (512, 8192, 1024, 0), (300, 4096, 4096, 0), (128, 2048, 2048, 1), (256, 4096, 1056, 0)]
+    assert [c for c in kernel if not L._pays(*c)] == [] and [c for c in gemm if L._pays(*c)] == []
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_project_is_the_kernel_or_torch(gpu):
+    for M, N, K, pays in ((128, 4096, 1024, True), (128, 1024, 3072, False)):
+        x, w = _xw((M,), N, K, torch.bfloat16, M)
+        assert torch.equal(L.project(x, w), L.linear(x, w) if pays else F.linear(x, w))
+        z = L.swiglu_project(x, w)
+        assert torch.equal(z, L.swiglu_linear(x, w)) if pays else z is None

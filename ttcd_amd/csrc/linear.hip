@@ -2,8 +2,9 @@
 //
 // The projections of a short prompt or of a follow-up of a few tokens read
 // each weight once for a handful of rows: they are bound by that read and by
-// their launches. A library GEMM costs ~17 us of host time per call here
+// their launches. A library GEMM costs ~19 us of host time per call here
 // (its choice of kernel is made again every time), more than the kernel runs.
+// Which of the two a call takes is decided by shape in linear.py (_pays).
 //
 // A workgroup owns 16 rows of W (16 gate and the 16 matching up rows in the
 // SwiGLU form) and up to 64 rows of x; its 8 wavefronts split K in steps of
@@ -138,11 +139,11 @@ __global__ __launch_bounds__(kLinWaves * 64) void linear_rows_kernel(LinearArgs 
 // Small tiles, because a call of a few hundred rows has few: 4096 x 1024, 300
 // rows, is 320 of them. A step then moves 16 KiB into LDS and 32 KiB out for
 // 16 MFMAs, and that LDS traffic bounds it (0.26 us a step; a 4-step ring is no
-// faster). Kernel time / library's (us): 4096 x 1024 128 rows 6.6 / 9.3, 512
-// rows 9.2 / 10.5, 1000 rows 17 / 13; 6144 x 1024 300 rows 9.4 / 10.5, 512
-// rows 13.9 / 13.3; 1024 x 3072 128 rows 13.0 / 8.3, 512 rows 13.1 / 12.3 (one
-// group of wavefronts 14.5). A library call costs 17 us of host time beside
-// it, a call of this kernel 4.
+// faster). Kernel / library (us, weights not in a cache): 4096 x 1024 128 rows
+// 7.7 / 12.5, 512 rows 11.2 / 13.1; 6144 x 1024 300 rows 11.2 / 13.3, 512 rows
+// 16.4 / 15.2; 1024 x 3072 128 rows 16.4 / 9.8, 512 rows 15.9 / 15.1. The last
+// shape's chain of 24 steps on 32 to 128 CUs is what the library shortens by
+// splitting K over workgroups.
 constexpr int kTileRows = 64;
 constexpr int kTileK = 64;
 constexpr int kRowBytes = kTileK * 2;

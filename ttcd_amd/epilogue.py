@@ -30,7 +30,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib
-from .linear import linear
+from .linear import project
 
 _DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16,
        torch.float32: _lib.DTYPE_F32}
@@ -166,8 +166,8 @@ def fused_attn_epilogue(o_proj: torch.nn.Linear, mlp_norm, o_t: torch.Tensor,
     if getattr(mlp_norm, "bias", None) is not None:
         raise NotImplementedError("fused_attn_epilogue: RMSNorm with bias")
     stacked = _stacked(o_t, o_s)
-    # one GEMM, or for few rows the kernel
-    proj = (linear(stacked, o_proj.weight) if o_proj.bias is None
+    # one GEMM, or the kernel where it is the faster
+    proj = (project(stacked, o_proj.weight) if o_proj.bias is None
             else F.linear(stacked, o_proj.weight, o_proj.bias))
     rows = B * T
     a_t = proj[:rows].view(B, T, -1)

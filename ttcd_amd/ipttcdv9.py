@@ -85,7 +85,7 @@ from . import attn as _attn
 from . import epilogue as _epi
 from . import prologue as _pro
 from . import ttt as _ttt
-from .linear import linear
+from .linear import project
 
 # configs/ipttcd/ipttcdv9_qwen3_0.6B_ct_64k_v2_swa8k.json (the config-5 model)
 QWEN3_06B_SWA8K = {
@@ -299,7 +299,7 @@ class IPTTCDv9Prefill:
         c, w = self.cfg, self.w
         B, T, _ = x.shape
         Hq, Hkv, D = self.Hq, self.Hkv, self.D
-        qkv = linear(x, self.qkv_w[i]).view(B, T, Hq + 2 * Hkv, D)
+        qkv = project(x, self.qkv_w[i]).view(B, T, Hq + 2 * Hkv, D)
         q, k, v = qkv.split((Hq, Hkv, Hkv), 2)
         p = f"model.layers.{i}.attn."
         cos, sin = ctx.tables if ctx.tables is not None else self.tables(ctx.offset + T)
@@ -417,7 +417,7 @@ class IPTTCDv9Prefill:
                              scan="kernel" if self.fuse_extra else "torch")
         else:
             o = self._teacher_attention(q, k, v, ctx)
-            a = linear(self._gate(i, xa, o), o_w)
+            a = project(self._gate(i, xa, o), o_w)
             x, residual = _epi.rmsnorm(a, w[p + "mlp_norm.weight"], eps, residual=residual)
             y = _ttt.swiglu_mlp(x, self.gu_w[i], w[p + "mlp.down_proj.weight"])
         return residual, y

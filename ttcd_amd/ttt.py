@@ -22,7 +22,7 @@ import torch
 import torch.nn.functional as F
 
 from . import _lib
-from .linear import linear, swiglu_linear
+from .linear import project, swiglu_project
 
 _DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16,
        torch.float32: _lib.DTYPE_F32}
@@ -78,12 +78,12 @@ def swiglu_mlp(x: torch.Tensor, gate_up_w: torch.Tensor, down_w: torch.Tensor) -
     """fla's swiglu_linear(gate_proj(x), up_proj(x), down_proj.weight)
     (custom_models/ipttcd/modeling_ipttcdv9.py:253-255; activations.py:508-540)
     with gate_proj and up_proj as one GEMM over the stacked (2*I, H) weight."""
-    z = swiglu_linear(x, gate_up_w)
+    z = swiglu_project(x, gate_up_w)
     if z is None:
         I = gate_up_w.shape[0] // 2
-        gu = linear(x, gate_up_w)
+        gu = project(x, gate_up_w)
         z = swiglu(gu[..., :I], gu[..., I:])
-    return linear(z, down_w)
+    return project(z, down_w)
 
 
 def _conv_weights(conv_t: torch.Tensor | None, conv_s: torch.Tensor | None, I: int):
