@@ -91,3 +91,20 @@ def test_project_is_the_kernel_or_torch(gpu):
         assert torch.equal(L.project(x, w), L.linear(x, w) if pays else F.linear(x, w))
         z = L.swiglu_project(x, w)
         assert torch.equal(z, L.swiglu_linear(x, w)) if pays else z is None
+
+
+@pytest.mark.gpu
+@torch.inference_mode()
+def test_autocast_casts(gpu):
+    """In an autocast region of another dtype the products are torch's, cast as
+    F.linear casts them; in one of the operands' own dtype nothing is cast."""
+    x, w = _xw((8,), 64, 64, torch.bfloat16, 3)
+    down = w[:, :32].contiguous()
+    with torch.autocast("cuda", torch.float16):
+        want = F.linear(x, w)
+        assert want.dtype == torch.float16 and torch.equal(L.project(x, w), want)
+        assert L.swiglu_project(x, w) is None
+        z = ttt.swiglu(want[:, :32], want[:, 32:])
+        assert torch.equal(ttt.swiglu_mlp(x, w, down), F.linear(z, down))
+    with torch.autocast("cuda", torch.bfloat16):
+        assert L._rows_for_kernel(x, w) == 8

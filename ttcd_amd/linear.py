@@ -29,6 +29,8 @@ def _rows_for_kernel(x: torch.Tensor, w: torch.Tensor) -> int:
             or w.shape[0] > MAX_COLS or w.shape[0] < 1
             or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
             or fwAD._current_level >= 0  # tangents are torch's to carry
+            # and so are autocast's casts
+            or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype)
             or not x.is_contiguous() or not w.is_contiguous()
             or x.data_ptr() % 16 or w.data_ptr() % 16):
         return 0
