@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import conv_ref
-from ttcd_amd import ttt
+from ttcd_amd import _lib, ttt
 
 pytestmark = pytest.mark.gpu
 
@@ -143,3 +143,32 @@ def test_swiglu_of_every_gate(gpu, dtype, u):
     assert torch.equal(got[~finite & ~want.isnan()], rounded[~finite & ~want.isnan()])
     w = want[finite].double()
     assert ((got[finite].double() - w).abs() <= (unit + 2.0 ** -20) * w.abs() + least).all()
+
+
+def _mlp_weights(I=32, H=64, conv_device="cuda"):
+    g = torch.Generator().manual_seed(I)
+    r = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16)  # noqa: E731
+    return ttt.TttMlpWeights(r(2 * I, H).cuda(), r(H, I).cuda(), r(H, H).cuda(),
+                             r(I, 1, 5).to(conv_device), r(I, 1, 5).to(conv_device), r(H).cuda())
+
+
+@pytest.mark.parametrize("L", [8, 40])
+def test_one_chunk_refuses_what_several_do(gpu, L):
+    """A prompt of one chunk reads neither the convs nor the update, and refuses the
+    same weights as a longer one: a width that swiglu does not take, convs on the CPU,
+    a gradient; empty batches are refused where a kernel would be launched."""
+    x = torch.randn(1, L, 64, generator=torch.Generator().manual_seed(L)).to(torch.bfloat16).cuda()
+    call = lambda w, **kw: ttt.ttt_mlp(x, x, w, chunk=16, lr=0.3, update_every=4, **kw)  # noqa: E731
+    with torch.no_grad():
+        for fused in (True, False):
+            with pytest.raises(_lib.TTCDError):
+                call(_mlp_weights(I=20), fused=fused)
+            for conv in ("kernel", "stock"):
+                with pytest.raises((ValueError, RuntimeError)):
+                    call(_mlp_weights(conv_device="cpu"), fused=fused, conv=conv)
+        with pytest.raises(_lib.TTCDError):
+            ttt.swiglu_mlp(x, _mlp_weights(I=20).gate_up, _mlp_weights(I=20).down)
+    w = _mlp_weights()
+    w.down.requires_grad_()
+    with pytest.raises(RuntimeError):
+        call(w)

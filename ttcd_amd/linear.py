@@ -111,8 +111,9 @@ def project(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def swiglu_project(x: torch.Tensor, gate_up: torch.Tensor) -> torch.Tensor | None:
-    """swiglu_linear where it is faster than the GEMM and a swiglu launch, else None."""
-    rows = _rows_for_kernel(x, gate_up) if gate_up.shape[0] % 2 == 0 else 0
+    """swiglu_linear where it is faster than the GEMM and a swiglu launch, else None:
+    also for the widths that swiglu refuses (no multiple of 8), whatever the rows."""
+    rows = _rows_for_kernel(x, gate_up) if gate_up.shape[0] % 16 == 0 else 0
     if rows and _pays(rows, gate_up.shape[0], gate_up.shape[1], True):
         return _run(x, gate_up, rows, gate_up.shape[0] // 2, 1)
     return None

@@ -329,6 +329,7 @@ def ttt_mlp(x: torch.Tensor, t: torch.Tensor, w: TttMlpWeights, *, chunk: int, l
     t = t.reshape(B, L, H).contiguous()
     if nchunk == 1:
         # no update: the plain MLP on the teacher's rows
+        _check_gpu("ttt_mlp", conv_t=w.conv_t, conv_s=w.conv_s, down=w.down)
         if fused and conv == "kernel" and _conv_weights(w.conv_t, w.conv_s, I)[2] > 8:
             raise _lib.TTCDError(_lib.TTCD_ERR_UNSUPPORTED, "conv kernel size must be in 1..8")
         return swiglu_mlp(x, w.gate_up, w.down)
