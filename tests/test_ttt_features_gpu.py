@@ -172,3 +172,17 @@ def test_one_chunk_refuses_what_several_do(gpu, L):
     w.down.requires_grad_()
     with pytest.raises(RuntimeError):
         call(w)
+
+
+@pytest.mark.parametrize("L", [8, 40])
+@torch.inference_mode()
+def test_empty_batches(gpu, L):
+    """No sequence: an empty result by torch's operations, refused where a kernel
+    would be launched."""
+    x = torch.empty(0, L, 64, dtype=torch.bfloat16, device=gpu)
+    call = lambda **kw: ttt.ttt_mlp(x, x, _mlp_weights(), chunk=16, lr=0.3, update_every=4, **kw)  # noqa: E731
+    for kw in (dict(), dict(fused=False), dict(scan="torch")):
+        with pytest.raises(ValueError):
+            call(**kw)
+    out = call(fused=False, conv="stock", scan="torch")
+    assert out.shape == (0, L, 64) and out.dtype == torch.bfloat16

@@ -327,6 +327,11 @@ def ttt_mlp(x: torch.Tensor, t: torch.Tensor, w: TttMlpWeights, *, chunk: int, l
         raise ValueError(f"ttt_mlp: need two matching non-empty (B, L, H) inputs, got "
                          f"{tuple(x.shape)} {dt}, {tuple(t.shape)} {t.dtype}")
     t = t.reshape(B, L, H).contiguous()
+    if B == 0:
+        if (conv == "kernel" and (fused or w.conv_t is not None or w.conv_s is not None)
+                or scan == "kernel" and nchunk > 1):
+            raise ValueError("ttt_mlp: the kernels need at least one sequence")
+        return torch.empty(0, L, H, dtype=dt, device=dev)
     if nchunk == 1:
         # no update: the plain MLP on the teacher's rows
         _check_gpu("ttt_mlp", conv_t=w.conv_t, conv_s=w.conv_s, down=w.down)
