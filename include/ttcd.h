@@ -386,13 +386,14 @@ ttcd_status ttcd_swiglu_fwd(const void* gate, const void* up, void* out,
                             ttcd_dtype dtype, void* stream);
 
 /*
- * y = x w^T for few rows (a short prompt's projections, the logits of the
- * last tokens): x (M, K) with row stride x_stride, w (N, K) contiguous, y
- * (M, N) contiguous; summed in fp32, rounded once. swiglu != 0: w (2N, K) is
- * the stacked gate | up weight and y the SwiGLU of the two products, each
- * rounded to dtype first, as ttcd_swiglu_fwd of the product would be.
- * K % 32 == 0, x_stride % 8 == 0; any M, meant for up to a few hundred rows
- * (more than 64 take 64 x 64 tiles when K % 64 == 0).
+ * y = x w^T for few rows (a short prompt's projections): x (M, K) with row
+ * stride x_stride, w (N, K) contiguous, y (M, N) contiguous; summed in fp32,
+ * rounded once. swiglu != 0: w (2N, K) is the stacked gate | up weight and y
+ * the SwiGLU of the two products, each rounded to dtype first, as
+ * ttcd_swiglu_fwd of the product would be. K % 32 == 0, x_stride % 8 == 0; x and
+ * w 16-byte aligned, y as its elements are (8 bytes and N % 4 == 0 make wider
+ * stores). Any M, meant for up to a few hundred rows (more than 64 take 64 x 64
+ * tiles when K % 64 == 0).
  */
 ttcd_status ttcd_linear_rows_fwd(const void* x, int64_t x_stride, const void* w, void* y, int M,
                                  int N, int K, int swiglu, ttcd_dtype dtype, void* stream);

@@ -108,3 +108,28 @@ def test_autocast_casts(gpu):
         assert torch.equal(ttt.swiglu_mlp(x, w, down), F.linear(z, down))
     with torch.autocast("cuda", torch.bfloat16):
         assert L._rows_for_kernel(x, w) == 8
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,glu", [
+    (5, 48, 96, 0), (64, 40, 256, 1), (65, 64, 128, 0), (130, 68, 192, 1), (515, 132, 64, 0),
+    (600, 36, 96, 0)])
+@pytest.mark.parametrize("shift", [0, 1, 4])
+@torch.inference_mode()
+def test_strided_rows_and_any_output_address(gpu, M, N, K, glu, shift):
+    """The C entry on a column slice of a wider x, more than MAX_ROWS rows among
+    them, and on outputs at any element: the bits of the same rows packed,
+    nothing written beside them."""
+    wide, w = _xw((M, 3), N * (1 + glu), K, torch.bfloat16, M + N)
+    x = wide[:, 1]
+    want = L._run(x.contiguous(), w, M, N, glu)
+    flat = torch.full((M * N + shift + 64,), 3.0, dtype=torch.bfloat16, device=gpu)
+    _lib.check(_lib.lib().ttcd_linear_rows_fwd(
+        x.data_ptr(), x.stride(0), w.data_ptr(), flat[shift:].data_ptr(), M, N, K, glu,
+        _lib.DTYPE_BF16, _lib.stream(x)))
+    assert torch.equal(flat[shift:shift + M * N].view(M, N), want)
+    assert (flat[:shift] == 3.0).all() and (flat[shift + M * N:] == 3.0).all()
+    if not glu:
+        exact = x.double() @ w.double().T
+        limit = 2.0 ** -8 * exact.abs() + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+        assert ((want.double() - exact).abs() <= limit).all()

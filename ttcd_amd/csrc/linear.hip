@@ -280,6 +280,7 @@ __global__ __launch_bounds__(256 * KS) void linear_tile_kernel(LinearArgs a) {
   const int m = m0 + wm * 32 + row;
   if (m >= a.M) return;
   T* y = static_cast<T*>(a.y) + (int64_t)m * a.N;
+  const bool wide = a.N % 4 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 7u) == 0;
 #pragma unroll
   for (int g = 0; g < 4; ++g) {
     const int n = n0 + wn * 32 + 8 * g + 4 * half;
@@ -295,7 +296,7 @@ __global__ __launch_bounds__(256 * KS) void linear_tile_kernel(LinearArgs a) {
                      static_cast<float>(round_to<T>(acc[NT - 1][4 * g + e])));
       v.e[e] = round_to<T>(f);
     }
-    if (n + 4 <= a.N && a.N % 4 == 0) {
+    if (wide && n + 4 <= a.N) {
       *reinterpret_cast<u32x2*>(y + n) = v.raw;
     } else {
 #pragma unroll
