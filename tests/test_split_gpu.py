@@ -14,7 +14,8 @@ import pytest
 import torch
 
 from conftest import make_qkv
-from ttcd_amd import _lib, fused_dual_window_attn, window_attn
+from ttcd_amd import (_lib, band_attn, fused_dual_window_attn, lse_dual_window_attn,
+                      window_attn)
 
 DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}
 
@@ -147,3 +148,29 @@ def test_near_and_far_scores_far_apart(gpu, Tq, Tk, ws, near, far, H, HK, D, dty
         _close(g, w, 1.02 * window_attn(q, k, v.abs(), W).float(), dtype, name)
     for g, w in ((got[2], want[2]), (got[3], want[3])):
         assert ((g - w).abs() <= 1e-5 + 2.0 ** -21 * w.abs()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,Tq,Tk,H,HK,D,wt,ws", [
+    (1, 300, 8491, 16, 8, 128, 8192, 4736), (2, 33, 5000, 15, 5, 64, -1, 4736)])
+@torch.inference_mode()
+def test_rows_that_are_not_split_have_the_bits_of_the_whole_prompt(gpu, B, Tq, Tk, H, HK, D, wt, ws):
+    """split_keys=False on calls that would be split: the last rows of the call on the
+    whole prompt, bit for bit; the LSE variant's student likewise."""
+    qf, k, v = make_qkv(batch=B, seqlen=Tk, heads=H, kv_heads=HK, head_dim=D, seed=Tk)
+    q = qf[:, Tk - Tq:]
+    hi = wt if wt > 0 else Tk
+    for lo, mid, top in ((0, ws, hi), (0, hi, hi), (0, ws, ws), (16, hi, hi)):
+        assert _bytes(B, Tq, Tk, H, HK, D, lo, mid, top) > 0
+    kw = dict(return_lse=True, split_keys=False)
+    for got, want in zip(fused_dual_window_attn(q, k, v, wt, ws, **kw),
+                         fused_dual_window_attn(qf, k, v, wt, ws, return_lse=True)):
+        rows = want[..., Tk - Tq:] if want.dim() == 3 else want[:, Tk - Tq:]
+        assert torch.equal(got, rows)
+    for lo, top in ((0, hi), (16, hi)):
+        o, lse = band_attn(q, k, v, lo, top, **kw)
+        wo, wl = band_attn(qf, k, v, lo, top, return_lse=True)
+        assert torch.equal(o, wo[:, Tk - Tq:]) and torch.equal(lse, wl[..., Tk - Tq:])
+    student = window_attn(q, k, v, ws, split_keys=False)
+    assert torch.equal(lse_dual_window_attn(q, k, v, wt, ws)[1], student)
+    assert torch.equal(window_attn(q[:1], k[:1], v[:1], ws, split_keys=False), student[:1])

@@ -82,12 +82,12 @@ def _ready(t: torch.Tensor) -> torch.Tensor:
 
 
 def _split_workspace(q: torch.Tensor, Tk: int, HK: int, lo: int, mid: int, hi: int,
-                     rescale: float):
+                     rescale: float, split_keys: bool):
     """(workspace or None, its bytes) for a cached prefill that the kernels would
     split over keys (ttcd_attn_kv_workspace_bytes); the caller keeps it until
     the call is launched."""
     B, T, H, D = q.shape
-    if T >= Tk:
+    if T >= Tk or not split_keys:
         return None, 0
     n = _lib.lib().ttcd_attn_kv_workspace_bytes(B, T, Tk, H, HK, D, lo, mid, hi, rescale)
     return (torch.empty(n, dtype=torch.uint8, device=q.device) if n else None), n
@@ -99,7 +99,8 @@ def _lse_ptr(t):
 
 def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
                            window_teacher: int, window_student: int, block_n: int = 64,
-                           *, return_lse: bool = False, exact_max: bool = False):
+                           *, return_lse: bool = False, exact_max: bool = False,
+                           split_keys: bool = True):
     """Returns (o_teacher, o_student) of one pass over K/V.
 
     Same call as profiling/fused_dual_attn.py:244: q (B, T, H, D), k/v
@@ -118,6 +119,8 @@ def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     275-293 asks of this call (a strict xfail for the reference kernel). Few
     queries over a long window are split over the keys, in a workspace
     allocated here: such rows agree with the unsplit call's to rounding.
+    ``split_keys=False`` never splits: a row then has the same bits in every
+    batch and however its prompt is cut into calls.
     """
     Tk = k.shape[1] if isinstance(k, torch.Tensor) and k.dim() == 4 else q.shape[1]
     if window_teacher is None or window_teacher < 0:
@@ -138,7 +141,7 @@ def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         lse_s = torch.empty(B, H, T, device=q.device, dtype=torch.float32)
     wt, ws = int(min(window_teacher, 2**31 - 1)), int(min(window_student, 2**31 - 1))
     rescale = _rescale(exact_max)
-    work, nbytes = _split_workspace(q, k.shape[1], HK, 0, ws, wt, rescale)
+    work, nbytes = _split_workspace(q, k.shape[1], HK, 0, ws, wt, rescale, split_keys)
     L = _lib.lib()
     _lib.check(L.ttcd_dual_window_attn_kv_ws_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), ot.data_ptr(), os_.data_ptr(),
@@ -152,12 +155,13 @@ def fused_dual_window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
 
 
 def band_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, band_lo: int, band_hi: int,
-              *, return_lse: bool = False, exact_max: bool = False):
+              *, return_lse: bool = False, exact_max: bool = False, split_keys: bool = True):
     """Causal attention over keys j with band_lo <= i - j < band_hi.
 
     (0, W) is flash_attn_func(q, k, v, causal=True, window_size=(W-1, 0));
     (WS, WT) is the far band of the LSE variant on unshifted tensors. Rows
-    whose band is empty get o = 0 and lse = -inf.
+    whose band is empty get o = 0 and lse = -inf. ``split_keys`` as in
+    fused_dual_window_attn.
     """
     B, T, H, HK, D = _check_qkv(q, k, v, "band_attn")
     Tk = k.shape[1]
@@ -170,7 +174,7 @@ def band_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, band_lo: int, b
     lse = torch.empty(B, H, T, device=q.device, dtype=torch.float32) if return_lse else None
     lo, hi = int(min(band_lo, 2**31 - 1)), int(min(band_hi, 2**31 - 1))
     rescale = _rescale(exact_max)
-    work, nbytes = _split_workspace(q, Tk, HK, lo, hi, hi, rescale)
+    work, nbytes = _split_workspace(q, Tk, HK, lo, hi, hi, rescale, split_keys)
     L = _lib.lib()
     _lib.check(L.ttcd_band_attn_kv_ws_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), _lse_ptr(lse),
@@ -182,16 +186,18 @@ def band_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, band_lo: int, b
 
 
 def window_attn(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window: int | None,
-                *, return_lse: bool = False, exact_max: bool = False):
+                *, return_lse: bool = False, exact_max: bool = False, split_keys: bool = True):
     """flash_attn_func(q, k, v, causal=True, window_size=(window-1, 0)) on gfx950;
     window None or < 0 = full causal. The "two separate calls" comparator.
     With k / v longer than q (a cached prefill), the queries are the last Tq
-    positions (flash-attention's bottom-right alignment)."""
+    positions (flash-attention's bottom-right alignment); ``split_keys`` as in
+    fused_dual_window_attn."""
     T = k.shape[1] if isinstance(k, torch.Tensor) and k.dim() == 4 else q.shape[1]
     w = T if (window is None or window < 0) else window
     if w < 1:
         raise ValueError("window must be >= 1")
-    return band_attn(q, k, v, 0, w, return_lse=return_lse, exact_max=exact_max)
+    return band_attn(q, k, v, 0, w, return_lse=return_lse, exact_max=exact_max,
+                     split_keys=split_keys)
 
 
 def _check_varlen(q, k, v, cu_seqlens, max_seqlen, fn: str):
@@ -358,6 +364,6 @@ def lse_dual_window_attn_fa3(q, k, v, window_teacher: int, window_student: int):
 
 def lse_dual_window_attn_fa3_fast(q, k, v, window_teacher: int, window_student: int):
     """profiling/lse_dual_attn.py:134-160 (two band calls + one-pass merge kernel);
-    the student output is exactly the single-window call's output (to rounding
-    where that call is a cached prefill split over the keys)."""
+    the student output is exactly the single-window call's output (of window_attn
+    with split_keys=False, where a cached prefill would be split over the keys)."""
     return lse_dual_window_attn(q, k, v, window_teacher, window_student)

@@ -185,15 +185,20 @@ size_t split_part_bytes(int B, int Tq, int Hq, int D) {
 // of the CU's time when it shares it, a launch 8 to start and end, the sum 3
 // and its traffic at 5 TB/s. Over 14 shapes of 1 to 3000 queries the parts it
 // picks are within 1 % (mean) of the best of 1 to 32. A split has to promise
-// 13 %. Not split: calls whose queries are the whole sequence and sweeps of
-// up to 72 tiles, whose rows are the same bits however a prompt is cut into
-// calls, and the exact running max, which is the reference kernel's own
-// order of accumulation.
+// 13 %. Not split: calls whose queries are the whole sequence, the exact running
+// max, which is the reference kernel's own order of accumulation, and sweeps of up
+// to 72 tiles (windows of up to about 4500 keys). The last is no matter of speed:
+// rows of such calls keep the bits that the whole prompt's call gives them
+// (tests/test_kv_attn_gpu.py). Longer sweeps give that up, unless the caller
+// passes no workspace (split_keys=False in Python).
 //
-// Measured (us, whole -> split, window 8192 on 8191 cached keys), 16/8 heads
-// of 128: 1 query 127 -> 23, 64 128 -> 30, 300 128 -> 44, 600 131 -> 66, 1000
-// 131 -> 90, 2048 188 -> 173; 15/5 heads of 64: 1 query 97 -> 21, 500
-// 99 -> 40, 1000 99 -> 62.
+// Measured (us, whole -> split, on a full window of cached keys). Window 8192,
+// 16/8 heads of 128: 1 query 127 -> 23, 64 128 -> 30, 300 128 -> 43, 600
+// 131 -> 66, 1000 131 -> 89, 2048 188 -> 173; 15/5 heads of 64: 1 query
+// 97 -> 20, 500 99 -> 40, 1000 99 -> 62. What the line at 72 tiles leaves, 16/8
+// heads of 128: window 4096, 1 query 66 -> 18, 300 69 -> 33; 2048 35 -> 16 and
+// 39 -> 27; 1024 20 -> 13 and 24 -> 23; 15/5 heads of 64, window 4096: 51 -> 17 and
+// 53 -> 31.
 SplitPlan split_plan(int B, int Tq, int Tk, int Hq, int Hkv, int D, int lo, int mid, int hi,
                      float rescale_log2) {
   SplitPlan none, best;
