@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from oracle import attn_ref, ipttcdv9_ref as R
-from ttcd_amd import _lib, ipttcdv9 as M
+from ttcd_amd import _lib, ipttcdv9 as M, ttt
 
 TINY = dict(M.QWEN3_06B_SWA8K, hidden_size=256, num_hidden_layers=3, num_heads=4, num_kv_heads=2,
             head_dim=64, intermediate_size=512, vocab_size=1024, window_size=512,
@@ -280,12 +280,28 @@ def test_ttt_features_abi_rejects():
 
 
 def test_python_layers_refuse_cpu_tensors():
-    from ttcd_amd import epilogue, ttt
+    from ttcd_amd import epilogue
     x = torch.zeros(4, 64, dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="GPU"):
         epilogue.rmsnorm(x, torch.ones(64), 1e-6)
     with pytest.raises(ValueError, match="GPU"):
         ttt.swiglu(x, x)
+
+
+@pytest.mark.parametrize("L,chunk", [(8, -4), (8, -100), (1, -4)])
+def test_ttt_mlp_refuses_a_chunk_below_one(monkeypatch, L, chunk):
+    """Refused before any buffer is sized by it: no feature row is written that its
+    output does not have."""
+    def swiglu(gate, up, out=None):
+        assert out is None or out.shape == gate.shape, (out.shape, gate.shape)
+        return torch.zeros_like(gate) if out is None else out.zero_()
+
+    monkeypatch.setattr(ttt, "swiglu", swiglu)
+    w = ttt.TttMlpWeights(torch.randn(64, 16), torch.randn(16, 32), None, None, None, None)
+    x = torch.randn(1, L, 16)
+    for kw in (dict(fused=False, conv="stock", scan="torch"), dict()):
+        with pytest.raises(ValueError):
+            ttt.ttt_mlp(x, x, w, chunk=chunk, lr=0.3, update_every=2, **kw)
 
 
 def test_output_gate_config_rules():

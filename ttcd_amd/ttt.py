@@ -323,6 +323,8 @@ def ttt_mlp(x: torch.Tensor, t: torch.Tensor, w: TttMlpWeights, *, chunk: int, l
         raise ValueError(f"ttt_mlp: conv must be 'kernel' or 'stock', got {conv!r}")
     if scan not in ("kernel", "torch"):
         raise ValueError(f"ttt_mlp: scan must be 'kernel' or 'torch', got {scan!r}")
+    if C < 1:
+        raise ValueError(f"ttt_mlp: chunk must be >= 1, got {C}")
     if L < 1 or t.numel() != x.numel() or t.dtype != dt or t.device != dev:
         raise ValueError(f"ttt_mlp: need two matching non-empty (B, L, H) inputs, got "
                          f"{tuple(x.shape)} {dt}, {tuple(t.shape)} {t.dtype}")
