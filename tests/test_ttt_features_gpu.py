@@ -186,3 +186,14 @@ def test_empty_batches(gpu, L):
             call(**kw)
     out = call(fused=False, conv="stock", scan="torch")
     assert out.shape == (0, L, 64) and out.dtype == torch.bfloat16
+
+
+@torch.inference_mode()
+def test_swiglu_output_must_hold_the_result(gpu):
+    """An output of fewer elements, another dtype or device is refused before the
+    launch; one of another shape with the same rows is not."""
+    g = torch.zeros(4, 32, dtype=torch.bfloat16, device=gpu)
+    for out in (g.half(), g[:2], g[:, :16], g.cpu()):
+        with pytest.raises(ValueError):
+            ttt.swiglu(g, g, out=out)
+    assert ttt.swiglu(g, g, out=g.view(2, 2, 32)).shape == (2, 2, 32)
