@@ -155,10 +155,11 @@ def _mlp_weights(I=32, H=64, conv_device="cuda"):
 @pytest.mark.parametrize("L", [8, 40])
 def test_one_chunk_refuses_what_several_do(gpu, L):
     """A prompt of one chunk reads neither the convs nor the update, and refuses the
-    same weights as a longer one: a width that swiglu does not take, convs on the CPU,
-    a gradient; empty batches are refused where a kernel would be launched."""
+    same calls as a longer one: a width that swiglu does not take, convs on the CPU or
+    that a separate conv does not take, a gradient, an autocast region that casts the
+    operands."""
     x = torch.randn(1, L, 64, generator=torch.Generator().manual_seed(L)).to(torch.bfloat16).cuda()
-    call = lambda w, **kw: ttt.ttt_mlp(x, x, w, chunk=16, lr=0.3, update_every=4, **kw)  # noqa: E731
+    call = lambda w, t=x, **kw: ttt.ttt_mlp(x, t, w, chunk=16, lr=0.3, update_every=4, **kw)  # noqa: E731
     with torch.no_grad():
         for fused in (True, False):
             with pytest.raises(_lib.TTCDError):
@@ -168,10 +169,29 @@ def test_one_chunk_refuses_what_several_do(gpu, L):
                     call(_mlp_weights(conv_device="cpu"), fused=fused, conv=conv)
         with pytest.raises(_lib.TTCDError):
             ttt.swiglu_mlp(x, _mlp_weights(I=20).gate_up, _mlp_weights(I=20).down)
+        for conv, shape, dtype in (("kernel", (40, 1, 5), torch.bfloat16),
+                                   ("kernel", (32, 1, 70), torch.bfloat16),
+                                   ("stock", (40, 1, 5), torch.bfloat16),
+                                   ("stock", (32, 1, 5), torch.float32)):
+            w = _mlp_weights()
+            w.conv_s = torch.ones(shape, dtype=dtype, device=gpu)
+            with pytest.raises((ValueError, RuntimeError)):
+                call(w, fused=False, conv=conv, scan="torch")
+        down32 = _mlp_weights()
+        down32.down = down32.down.float()
+        for w, region in ((_mlp_weights(), torch.float16), (down32, torch.bfloat16)):
+            with torch.autocast("cuda", region), pytest.raises((ValueError, RuntimeError)):
+                call(w)
     w = _mlp_weights()
+    with pytest.raises(RuntimeError):
+        call(w, t=x.clone().requires_grad_())
     w.down.requires_grad_()
     with pytest.raises(RuntimeError):
         call(w)
+    if L <= 16:  # torch's own conv takes a gradient, and its result is not read
+        w = _mlp_weights()
+        w.conv_s.requires_grad_()
+        assert call(w, fused=False, conv="stock").shape == x.shape
 
 
 @pytest.mark.parametrize("L", [8, 40])

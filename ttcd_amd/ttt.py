@@ -112,6 +112,33 @@ def _conv_weights(conv_t: torch.Tensor | None, conv_s: torch.Tensor | None, I: i
     return ws, next((w.dtype for w in ws if w is not None), torch.float32), K or 1
 
 
+def _check_convs(w: TttMlpWeights, I: int, dt: torch.dtype, dev: torch.device, fused: bool,
+                 conv: str):
+    """Refuses the conv weights that the feature passes refuse, for a prompt of one
+    chunk, which runs none of them."""
+    if fused and conv == "kernel":
+        _check_gpu("ttt_mlp", conv_t=w.conv_t, conv_s=w.conv_s)
+        _, wdt, K = _conv_weights(w.conv_t, w.conv_s, I)
+        if wdt not in _DT or K > 8:
+            raise _lib.TTCDError(_lib.TTCD_ERR_UNSUPPORTED, "conv kernel size must be in 1..8, "
+                                 "its weights bf16, f16 or f32")
+        return
+    for cw in (w.conv_t, w.conv_s):
+        if cw is None:
+            continue
+        K = cw.reshape(I, -1).shape[1]
+        if cw.device != dev or K < 1:
+            raise ValueError(f"ttt_mlp: conv weights must be (I, K) on {dev}")
+        if conv == "stock":  # conv1d's operands share a dtype, unless autocast casts them
+            if cw.dtype != dt and not torch.is_autocast_enabled("cuda"):
+                raise ValueError(f"ttt_mlp: x is {dt}, a conv weight {cw.dtype}")
+        else:
+            _check_gpu("ttt_mlp", conv=cw)
+            if cw.dtype not in _DT or K > 64:
+                raise _lib.TTCDError(_lib.TTCD_ERR_UNSUPPORTED, "conv kernel size must be in "
+                                     "1..64, its weights bf16, f16 or f32")
+
+
 def ttt_features(gu_t: torch.Tensor, gu_s: torch.Tensor, conv_t: torch.Tensor | None,
                  conv_s: torch.Tensor | None, B: int, nchunk: int, chunk: int):
     """gu_t / gu_s: (B*nchunk*chunk, 2*I) gate|up rows of the teacher / student.
@@ -340,10 +367,13 @@ def ttt_mlp(x: torch.Tensor, t: torch.Tensor, w: TttMlpWeights, *, chunk: int, l
         return torch.empty(0, L, H, dtype=dt, device=dev)
     if nchunk == 1:
         # no update: the plain MLP on the teacher's rows
-        _check_gpu("ttt_mlp", conv_t=w.conv_t, conv_s=w.conv_s, down=w.down)
-        if fused and conv == "kernel" and _conv_weights(w.conv_t, w.conv_s, I)[2] > 8:
-            raise _lib.TTCDError(_lib.TTCD_ERR_UNSUPPORTED, "conv kernel size must be in 1..8")
-        return swiglu_mlp(x, w.gate_up, w.down)
+        _check_gpu("ttt_mlp", t=t, down=w.down)
+        _check_convs(w, I, dt, dev, fused, conv)
+        out = swiglu_mlp(x, w.gate_up, w.down)
+        if w.down.dtype != dt or out.dtype != dt:  # autocast casts what the updates do not
+            raise ValueError(f"ttt_mlp: x is {dt}, the down projection {w.down.dtype}, the "
+                             f"result {out.dtype}")
+        return out
     # The student's features are read by the updates, so never those of the
     # last chunk: its gate|up rows stop at the end of the last full one.
     upd = (nchunk - 1) * C
