@@ -217,3 +217,22 @@ def test_swiglu_output_must_hold_the_result(gpu):
         with pytest.raises(ValueError):
             ttt.swiglu(g, g, out=out)
     assert ttt.swiglu(g, g, out=g.view(2, 2, 32)).shape == (2, 2, 32)
+
+
+@pytest.mark.parametrize("L", [8, 16, 32, 40])
+@torch.inference_mode()
+def test_shapes_of_the_student_input(gpu, L):
+    """Whole chunks take the student's rows in any shape; a partial one takes the
+    sequences as they are, since other shapes were padded elsewhere and refused."""
+    r = lambda *s: torch.randn(*s, generator=torch.Generator().manual_seed(L)).to(torch.bfloat16).cuda()  # noqa: E731
+    call = lambda x, t: ttt.ttt_mlp(x, t, _mlp_weights(), chunk=16, lr=0.3, update_every=2)  # noqa: E731
+    x, t = r(2, L, 64), r(2, L, 64)
+    want = call(x, t)
+    assert torch.equal(call(x, t.view(1, 2, L, 64)), want)
+    assert torch.equal(call(x[:1], t[0]), call(x[:1], t[:1]))
+    for shape in ((2 * L, 64), (2 * L * 64,), (L, 2, 64), (2, 64, L)):
+        if L % 16:
+            with pytest.raises(ValueError):
+                call(x, t.reshape(shape))
+        else:
+            assert torch.equal(call(x, t.reshape(shape)), want)

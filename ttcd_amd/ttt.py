@@ -359,6 +359,9 @@ def ttt_mlp(x: torch.Tensor, t: torch.Tensor, w: TttMlpWeights, *, chunk: int, l
     if L < 1 or t.numel() != x.numel() or t.dtype != dt or t.device != dev:
         raise ValueError(f"ttt_mlp: need two matching non-empty (B, L, H) inputs, got "
                          f"{tuple(x.shape)} {dt}, {tuple(t.shape)} {t.dtype}")
+    if L % C and t.shape[-2:] != (L, H):  # whole chunks take any shape of these rows
+        raise ValueError(f"ttt_mlp: with a partial last chunk t must be (.., {L}, {H}), got "
+                         f"{tuple(t.shape)}")
     t = t.reshape(B, L, H).contiguous()
     if B == 0:
         if (conv == "kernel" and (fused or w.conv_t is not None or w.conv_s is not None)
