@@ -236,3 +236,14 @@ def test_shapes_of_the_student_input(gpu, L):
                 call(x, t.reshape(shape))
         else:
             assert torch.equal(call(x, t.reshape(shape)), want)
+
+
+@torch.inference_mode()
+def test_learning_rate_weight_is_a_vector(gpu):
+    """(H, 1) would give every token its rate too, one dimension deeper."""
+    x = torch.randn(1, 40, 64, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16).cuda()
+    w = _mlp_weights()
+    w.b_proj = w.b_proj[:, None]
+    for scan in ("kernel", "torch"):
+        with pytest.raises(ValueError):
+            ttt.ttt_mlp(x, x, w, chunk=16, lr=0.3, update_every=2, scan=scan)

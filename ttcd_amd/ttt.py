@@ -213,6 +213,8 @@ def _beta(t: torch.Tensor, b_proj: torch.Tensor, rows: int) -> torch.Tensor:
     """(t @ b_proj).sigmoid() of the first `rows` tokens of every sequence of t
     (B, L, H), each step rounded to the dtype (scanfuse.py:72-74): (B, rows)."""
     B, L, H = t.shape
+    if b_proj.dim() != 1:
+        raise ValueError(f"ttt_mlp: b_proj must be ({H},), got {tuple(b_proj.shape)}")
     if (H % 8 or t.data_ptr() % 16 or b_proj.shape != (H,) or not b_proj.is_contiguous()
             or b_proj.dtype != t.dtype or b_proj.device != t.device or b_proj.data_ptr() % 16):
         return torch.matmul(t[:, :rows], b_proj).sigmoid().contiguous()
