@@ -29,9 +29,15 @@ def test_what_is_split():
     n = _bytes(1, 300, 8491, 16, 8, 128, 0, 8192, 8192)
     assert n % one == 0 and 2 <= n // one <= 32
     assert _bytes(1, 300, 8491, 16, 8, 128, 0, 4096, -1) % one == 0
+    for call in ((1, 2048, 10239, 15, 5, 64, 0, 4096, 8192), (1, 4096, 12287, 4, 2, 64, 0, 4096, 8192)):
+        assert _bytes(*call) > 0, call
     for call in ((1, 8491, 8491, 16, 8, 128, 0, 8192, 8192),    # not cached
                  (1, 300, 4600, 16, 8, 128, 0, 4224, 4224),     # 4 KiB of keys, as one sweep
                  (1, 8000, 16191, 16, 8, 128, 0, 8192, 8192),   # fills the GPU
+                 # rows with a part of their window: the unsplit sweeps are the shorter
+                 (1, 11186, 27569, 4, 4, 128, 0, 27569, 27569),
+                 # one part with nearly all of the window
+                 (2, 4301, 9079, 4, 2, 64, 0, 7168, 9079), (3, 910, 9507, 15, 5, 64, 0, 8064, 9507),
                  (1, 300, 8491, 16, 7, 128, 0, 8192, 8192),     # not a call
                  (1, 300, 8491, 16, 8, 96, 0, 8192, 8192),
                  (1, 300, 8491, 16, 8, 128, 4, 4, 8)):

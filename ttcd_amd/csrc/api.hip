@@ -183,22 +183,25 @@ size_t split_part_bytes(int B, int Tq, int Hq, int D) {
 // parts end there). The rule is a model of the call's time in us, its rates
 // fitted to an MI355X: a slot takes `alone` with its CU to itself and `busy`
 // of the CU's time when it shares it, a launch 8 to start and end, the sum 3
-// and its traffic at 5 TB/s. Over 14 shapes of 1 to 3000 queries the parts it
-// picks are within 1 % (mean) of the best of 1 to 32. A split has to promise
-// 13 %. Not split: calls whose queries are the whole sequence, the exact running
-// max, which is the reference kernel's own order of accumulation, and sweeps of up
-// to 72 tiles (windows of up to about 4500 keys). The last is no matter of speed:
-// rows of such calls keep the bits that the whole prompt's call gives them
-// (tests/test_kv_attn_gpu.py). Longer sweeps give that up, unless the caller
-// passes no workspace (split_keys=False in Python).
+// and its traffic at 5 TB/s. A split has to promise 18 %: the model is up to that
+// far off where the CUs hold two or three workgroups. Of 2000 split calls drawn from 1
+// to 14000 queries on 100 to 32000 cached keys, 8 sets of heads and windows of 6000
+// to full, the geometric mean took 0.31 of its unsplit time and none
+// more than 1.08 of it. Not split: calls whose queries are the whole sequence, the
+// exact running max, which is the reference kernel's own order of accumulation,
+// and sweeps of up to 72 tiles (windows of up to about 4500 keys). The last is no
+// matter of speed: rows of such calls keep the bits that the whole prompt's call
+// gives them (tests/test_kv_attn_gpu.py). Longer sweeps give that up, unless the
+// caller passes no workspace (split_keys=False in Python).
 //
 // Measured (us, whole -> split, on a full window of cached keys). Window 8192,
-// 16/8 heads of 128: 1 query 127 -> 23, 64 128 -> 30, 300 128 -> 43, 600
-// 131 -> 66, 1000 131 -> 89, 2048 188 -> 173; 15/5 heads of 64: 1 query
-// 97 -> 20, 500 99 -> 40, 1000 99 -> 62. What the line at 72 tiles leaves, 16/8
-// heads of 128: window 4096, 1 query 66 -> 18, 300 69 -> 33; 2048 35 -> 16 and
-// 39 -> 27; 1024 20 -> 13 and 24 -> 23; 15/5 heads of 64, window 4096: 51 -> 17 and
-// 53 -> 31.
+// 16/8 heads of 128: 1 query 123 -> 24, 64 127 -> 30, 300 128 -> 42, 600
+// 128 -> 63, 1000 129 -> 86, 2048 183 -> 167; 15/5 heads of 64: 1 query
+// 95 -> 20, 500 98 -> 42, 1000 99 -> 60, 2048 106 -> 90. Not split by this rule:
+// 11186 queries on 16383 keys, 4/4 heads of 128, full causal (513; in two parts
+// 600). What the line at 72 tiles leaves, 16/8 heads of 128: window 4096, 1 query
+// 66 -> 18, 300 69 -> 33; 2048 35 -> 16 and 39 -> 27; 1024 20 -> 13 and 24 -> 23; 15/5
+// heads of 64, window 4096: 51 -> 17 and 53 -> 31.
 SplitPlan split_plan(int B, int Tq, int Tk, int Hq, int Hkv, int D, int lo, int mid, int hi,
                      float rescale_log2) {
   SplitPlan none, best;
@@ -212,21 +215,29 @@ SplitPlan split_plan(int B, int Tq, int Tk, int Hq, int Hkv, int D, int lo, int 
   const int64_t blocks = (Tk + span - 1) / span - (Tk - Tq) / span;
   const int64_t nwg = (int64_t)B * Hkv * (G / (ttcd::kWaveRows / rows)) * blocks;
   const double alone = D == 128 ? 0.95 : 0.70, busy = D == 128 ? 0.80 : 0.45;
-  const int cus = ttcd::kXcd * ttcd::kXcdCus;
-  auto model = [&](int parts) {
-    const double n = (double)((nwg * parts + cus - 1) / cus);
-    const double slots = (double)sweep / parts + (parts > 1 ? 1.5 : 0.0);
-    double t = 8.0 + slots * (alone > n * busy ? alone : n * busy);
+  const int cus = ttcd::kXcd * ttcd::kXcdCus, places = D == 128 ? 2 : 3;
+  // keys that the rows lack at their sequence's start, on average
+  const double first = Tk - Tq + 1, last = hi - 1;  // histories shorter than hi
+  const double missing =
+      first > last ? 0.0 : (last - first + 1) * (hi - 0.5 * (first + last)) / Tq;
+  const double mean = sweep - (missing < hi - lo ? missing : hi - lo) / ttcd::kBlockN;
+  // parts of at most `step` of the band's distances
+  auto model = [&](int parts, int step) {
+    const double n = (double)((nwg * parts + cus - 1) / cus), ends = parts > 1 ? 1.5 : 0.0;
+    const double longest = sweep * ((double)step / (hi - lo)) + ends;
+    // A workgroup that waits for a place is one of the long ones; parts much longer
+    // than the mean meet on a CU by chance.
+    const double each = (n > places && parts > 1 ? sweep : mean) / parts + ends;
+    const double chance = parts > 1 && longest > 1.5 * each ? longest - 1.5 * each : 0.0;
+    const double work = n * busy * (each + chance);
+    double t = 8.0 + (alone * longest > work ? alone * longest : work);
     if (parts > 1) t += 3.0 + 2.0 * parts * split_part_bytes(B, Tq, Hq, D) / 5e6;
     return t;
   };
-  double least = 0.87 * model(1);
+  double least = 0.82 * model(1, hi - lo);
   for (int p = 2; p <= 16 && sweep / p >= 4; ++p) {
     if (p * split_part_bytes(B, Tq, Hq, D) > kSplitMaxBytes) break;
-    const double t = model(p);
-    if (t >= least) continue;
-    least = t;
-    best = none;
+    SplitPlan sp;
     auto cut = [&](int width, int parts, int* n, int* step) {
       *step = ((width + parts - 1) / parts + ttcd::kBlockN - 1) / ttcd::kBlockN * ttcd::kBlockN;
       *n = (width + *step - 1) / *step;
@@ -234,8 +245,13 @@ SplitPlan split_plan(int B, int Tq, int Tk, int Hq, int Hkv, int D, int lo, int 
     const int far = hi - mid;
     int near_p = far > 0 ? (int)((int64_t)p * (mid - lo) / (hi - lo)) : p;
     near_p = near_p < 1 ? 1 : near_p;
-    cut(mid - lo, near_p, &best.near_parts, &best.near_step);
-    if (far > 0) cut(far, p - near_p > 1 ? p - near_p : 1, &best.far_parts, &best.far_step);
+    cut(mid - lo, near_p, &sp.near_parts, &sp.near_step);
+    if (far > 0) cut(far, p - near_p > 1 ? p - near_p : 1, &sp.far_parts, &sp.far_step);
+    const int step = sp.near_step > sp.far_step ? sp.near_step : sp.far_step;
+    const double t = model(sp.parts(), step < hi - lo ? step : hi - lo);
+    if (t >= least) continue;
+    least = t;
+    best = sp;
   }
   return best;
 }
