@@ -1243,14 +1243,15 @@ ttcd_status ttcd_attn_block_coverage(int npair, int nqb, int ngrp, int packed, i
                                      int64_t xcd_work[8]) {
   if (npair < 1 || nqb < 1 || ngrp < 1 || !counts || !xcd_work)
     return fail(TTCD_ERR_INVALID_ARGUMENT, "bad block coverage arguments");
-  const ttcd::BlockMap m = ttcd::make_block_map(npair, nqb, ngrp, packed != 0);
+  const ttcd::BlockMap m = 
+      ttcd::make_block_map(npair, packed & 1 ? 1 : npair, nqb, ngrp, packed == 1);
   for (int g = 0; g < m.launched(); ++g) {
     int pair, qb, grp;
     if (!m.locate(g, &pair, &qb, &grp)) continue;
     if (pair < 0 || pair >= npair || qb < 0 || qb >= nqb || grp < 0 || grp >= ngrp)
       return fail(TTCD_ERR_UNSUPPORTED, "block map error: id %d -> (%d, %d, %d)", g, pair, qb, grp);
     counts[((int64_t)pair * nqb + qb) * ngrp + grp] += 1;
-    xcd_work[g % ttcd::kXcd] += qb + 1;
+    xcd_work[g % ttcd::kXcd] += packed == 2 ? 1 : (int64_t)(qb + 1) * (packed & 1 ? pair + 1 : 1);
   }
   return ok();
 }

@@ -1046,8 +1046,9 @@ void attn_fwd_kernel(AttnArgs a) {
 template <int D, typename T, bool DUAL>
 hipError_t launch_typed(const AttnArgs& a, hipStream_t stream) {
   AttnArgs args = a;
-  args.map = make_block_map(a.B * a.Hkv, a.nqb, a.G / (kWaveRows / a.sched.rows),
-                            a.cu_seqlens != nullptr);
+  const bool packed = a.cu_seqlens != nullptr;
+  args.map = make_block_map(a.B * a.Hkv, packed ? a.Hkv : a.B * a.Hkv, a.nqb,
+                            a.G / (kWaveRows / a.sched.rows), packed);
   args.hkv = make_fast_div(a.Hkv);
   const int nwg = args.map.launched();
   // The sum-triggered lazy slot needs a second P^T buffer, which D = 64 has
@@ -1069,7 +1070,7 @@ hipError_t launch_typed(const AttnArgs& a, hipStream_t stream) {
 template <int D, typename T>
 hipError_t launch_parts(const AttnArgs& a, hipStream_t stream) {
   AttnArgs args = a;
-  args.map = make_block_map(a.B * a.Hkv * a.parts, a.nqb,
+  args.map = make_block_map(a.B * a.Hkv * a.parts, a.B * a.Hkv, a.nqb,
                             a.G / (kWaveRows / a.sched.rows), false);
   args.hkv = make_fast_div(a.Hkv);
   args.pairs = make_fast_div(a.B * a.Hkv);

@@ -308,8 +308,10 @@ TTCD_HD Band word_band(const Schedule& sc, uint32_t w) { return (w & kWordFar) ?
 // are dealt to the XCDs level by level: every XCD gets the same share of
 // every level of every head (of every packed sequence too), while the
 // workgroups of an item, which sweep nearly the same keys, share one L2.
-// With npair a multiple of 8 an XCD keeps whole heads; otherwise the deal
-// runs forth and back so that no XCD always gets the heavier items.
+// With npair a multiple of 8 the deal leaves an XCD whole heads; where these are
+// not alike (sequences of a packed call, parts of a split one) it starts one
+// XCD later every round. With another npair it runs forth and back, so that no
+// XCD always gets the heavier items.
 //
 // Why: one contiguous run of (head, block) per XCD leaves the XCDs unequal
 // when a head's run is split between them (causal heads, npair not a multiple
@@ -344,6 +346,10 @@ TTCD_HD FastDiv make_fast_div(int d) {
   return f;
 }
 
+// How the items go to the XCDs: always in the same direction, forth and back, or
+// from one XCD later every round (a mask of the round).
+enum BlockDeal : int { kDealForth = 0, kDealSnake = 1, kDealTurn = 7 << 1 };
+
 struct BlockMap {
   int nqb;               // query blocks per K/V head
   FastDiv npair, ngrp;   // K/V heads, workgroups per block
@@ -351,7 +357,7 @@ struct BlockMap {
   int seg;               // blocks per item
   int items;             // (levels) * npair
   int rounds;            // items per XCD, rounded up
-  int snake;             // the deal changes direction every round
+  int deal;
 
   TTCD_HD int per_xcd() const { return rounds * (int)per.d; }
   TTCD_HD int launched() const { return kXcd * per_xcd(); }
@@ -370,9 +376,11 @@ struct BlockMap {
   // The K/V head, query block and workgroup of the block that id g takes;
   // false when it takes none.
   TTCD_HD bool locate(int g, int* pair, int* qb, int* grp) const {
-    const int x = g % kXcd, r = rank(g / kXcd);
+    const int x = g % kXcd;
+    const int r = rank(g / kXcd);
     const int round = per.quot(r), in = r - round * (int)per.d;
-    const int item = round * kXcd + ((snake & round & 1) ? kXcd - 1 - x : x);
+    const int at = ((x + (round & deal >> 1)) & (kXcd - 1)) ^ (-(deal & round & 1) & (kXcd - 1));
+    const int item = round * kXcd + at;
     const int level = npair.quot(item);
     const int blk = ngrp.quot(in);
     *pair = item - level * (int)npair.d;
@@ -382,20 +390,24 @@ struct BlockMap {
   }
 };
 
-// Blocks per item. A fixed-length call whose heads are a multiple of the XCDs
+// Blocks per item. A fixed-length call whose heads (alike of them in a row sweep
+// alike: all, the ones of a sequence, or of a part) are a multiple of the XCDs
 // gives each XCD whole heads. Otherwise: when every workgroup starts at once
 // on a CU of its own, as few items as give every XCD one (the sweep of the
 // heaviest workgroup is then the call, and it is fastest when the workgroups
-// beside it fetch the same tiles); when they queue, 8 items per XCD, so that
-// its share differs by little, of at least 4 blocks (whose workgroups share
-// nearly all of their tiles) and at most 32 (about what an XCD runs at once).
+// beside it fetch the same tiles); when they queue, 8 items per XCD of at
+// least 4 blocks (whose workgroups share nearly all of their tiles) and at most
+// 32 (about what an XCD runs at once).
 //
 // Measured against one contiguous run per XCD (us, kernel time): packed
 // 12345 tokens in 9 sequences, 15/5 heads of 64, 153 -> 88; causal T = 8192,
 // 15/5 heads of 64, 230 -> 162, T = 4500 80.7 -> 67.9; 16/8 heads of 128,
 // T = 8192, 282 -> 271 and T = 4096 92.3 -> 87.2 (the order within an XCD
 // alone); 4/2 heads of 64, T = 4096, with 64 items instead of 8 50.6 -> 54.1.
-TTCD_HD BlockMap make_block_map(int npair, int nqb, int ngrp, bool packed) {
+// Parts dealt from one XCD later every round instead of a part to an XCD (us, call
+// time, full windows of cached keys): 2048 queries, 15/5 heads of 64, window 8192
+// 111 -> 92; 4096, 4/2 heads, 80 -> 60.
+TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool packed) {
   BlockMap m;
   m.nqb = nqb;
   m.npair = make_fast_div(npair);
@@ -404,13 +416,13 @@ TTCD_HD BlockMap make_block_map(int npair, int nqb, int ngrp, bool packed) {
   int seg = 32;
   auto few = [&](int items) { return (int64_t)npair * ((nqb + seg - 1) / seg) < items; };
   while (seg > 1 && few(queued && seg > 4 ? 8 * kXcd : kXcd)) seg /= 2;
-  if (!packed && npair % kXcd == 0) seg = nqb;
+  if (!packed && alike % kXcd == 0) seg = nqb;
   const int levels = (nqb + seg - 1) / seg;
   m.seg = (nqb + levels - 1) / levels;
   m.per = make_fast_div(m.seg * ngrp);
   m.items = levels * npair;
   m.rounds = (m.items + kXcd - 1) / kXcd;
-  m.snake = npair % kXcd != 0;
+  m.deal = npair % kXcd != 0 ? kDealSnake : alike % kXcd != 0 ? kDealTurn : kDealForth;
   return m;
 }
 
