@@ -1244,7 +1244,7 @@ ttcd_status ttcd_attn_block_coverage(int npair, int nqb, int ngrp, int packed, i
   if (npair < 1 || nqb < 1 || ngrp < 1 || !counts || !xcd_work)
     return fail(TTCD_ERR_INVALID_ARGUMENT, "bad block coverage arguments");
   const ttcd::BlockMap m = 
-      ttcd::make_block_map(npair, packed & 1 ? 1 : npair, nqb, ngrp, packed == 1);
+      ttcd::make_block_map(npair, packed & 1 ? 1 : npair, nqb, ngrp, packed == 1, packed == 2);
   for (int g = 0; g < m.launched(); ++g) {
     int pair, qb, grp;
     if (!m.locate(g, &pair, &qb, &grp)) continue;

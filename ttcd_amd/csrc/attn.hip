@@ -1048,7 +1048,8 @@ hipError_t launch_typed(const AttnArgs& a, hipStream_t stream) {
   AttnArgs args = a;
   const bool packed = a.cu_seqlens != nullptr;
   args.map = make_block_map(a.B * a.Hkv, packed ? a.Hkv : a.B * a.Hkv, a.nqb,
-                            a.G / (kWaveRows / a.sched.rows), packed);
+                            a.G / (kWaveRows / a.sched.rows), packed,
+                            !packed && even_rows(a.T, a.q_off, a.sched.p2.hi));
   args.hkv = make_fast_div(a.Hkv);
   const int nwg = args.map.launched();
   // The sum-triggered lazy slot needs a second P^T buffer, which D = 64 has
@@ -1070,8 +1071,10 @@ hipError_t launch_typed(const AttnArgs& a, hipStream_t stream) {
 template <int D, typename T>
 hipError_t launch_parts(const AttnArgs& a, hipStream_t stream) {
   AttnArgs args = a;
+  const int far = a.near_parts < a.parts ? a.far_step : a.near_step;
   args.map = make_block_map(a.B * a.Hkv * a.parts, a.B * a.Hkv, a.nqb,
-                            a.G / (kWaveRows / a.sched.rows), false);
+                            a.G / (kWaveRows / a.sched.rows), false,
+                            even_rows(a.T, a.q_off, a.sched.p2.hi) && far == a.near_step);
   args.hkv = make_fast_div(a.Hkv);
   args.pairs = make_fast_div(a.B * a.Hkv);
   hipLaunchKernelGGL((attn_fwd_kernel<D, T, false, D == 128, true>), dim3(args.map.launched()),

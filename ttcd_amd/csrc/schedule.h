@@ -316,7 +316,9 @@ TTCD_HD Band word_band(const Schedule& sc, uint32_t w) { return (w & kWordFar) ?
 // Why: one contiguous run of (head, block) per XCD leaves the XCDs unequal
 // when a head's run is split between them (causal heads, npair not a multiple
 // of 8) or when packed sequences differ in length; the call then waits for
-// one XCD.
+// one XCD. Where all workgroups sweep alike, or each has a CU to itself, a run
+// per XCD is even to one workgroup, and items are not: such calls take runs
+// when the deal would leave an XCD too many.
 //
 // Within an XCD the workgroups start heaviest first, except that the second
 // one of each CU is taken so that a CU's two add up to about the same sweep:
@@ -347,19 +349,20 @@ TTCD_HD FastDiv make_fast_div(int d) {
 }
 
 // How the items go to the XCDs: always in the same direction, forth and back, or
-// from one XCD later every round (a mask of the round).
-enum BlockDeal : int { kDealForth = 0, kDealSnake = 1, kDealTurn = 7 << 1 };
+// from one XCD later every round (a mask of the round). Or no items: one run of
+// workgroups per XCD.
+enum BlockDeal : int { kDealForth = 0, kDealSnake = 1, kDealTurn = 7 << 1, kDealRuns = 16 };
 
 struct BlockMap {
   int nqb;               // query blocks per K/V head
   FastDiv npair, ngrp;   // K/V heads, workgroups per block
-  FastDiv per;           // workgroups per item
-  int seg;               // blocks per item
-  int items;             // (levels) * npair
-  int rounds;            // items per XCD, rounded up
+  FastDiv per;           // workgroups per item (runs: nqb)
+  int seg;               // blocks per item (runs: workgroups per run)
+  int items;             // (levels) * npair (runs: the XCDs whose run has one more)
+  int rounds;            // items per XCD, rounded up (runs: workgroups, rounded up)
   int deal;
 
-  TTCD_HD int per_xcd() const { return rounds * (int)per.d; }
+  TTCD_HD int per_xcd() const { return deal == kDealRuns ? rounds : rounds * (int)per.d; }
   TTCD_HD int launched() const { return kXcd * per_xcd(); }
 
   // Position in the heaviest-first order of an XCD's n workgroups of its
@@ -377,6 +380,14 @@ struct BlockMap {
   // false when it takes none.
   TTCD_HD bool locate(int g, int* pair, int* qb, int* grp) const {
     const int x = g % kXcd;
+    if (deal == kDealRuns) {
+      const int i = g / kXcd, at = x * seg + (x < items ? x : items) + i;
+      const int row = ngrp.quot(at);
+      *grp = at - row * (int)ngrp.d;
+      *pair = per.quot(row);
+      *qb = nqb - 1 - (row - *pair * nqb);
+      return i < seg + (x < items ? 1 : 0);
+    }
     const int r = rank(g / kXcd);
     const int round = per.quot(r), in = r - round * (int)per.d;
     const int at = ((x + (round & deal >> 1)) & (kXcd - 1)) ^ (-(deal & round & 1) & (kXcd - 1));
@@ -397,7 +408,8 @@ struct BlockMap {
 // heaviest workgroup is then the call, and it is fastest when the workgroups
 // beside it fetch the same tiles); when they queue, 8 items per XCD of at
 // least 4 blocks (whose workgroups share nearly all of their tiles) and at most
-// 32 (about what an XCD runs at once).
+// 32 (about what an XCD runs at once). even: all blocks sweep about as many
+// tiles.
 //
 // Measured against one contiguous run per XCD (us, kernel time): packed
 // 12345 tokens in 9 sequences, 15/5 heads of 64, 153 -> 88; causal T = 8192,
@@ -407,12 +419,21 @@ struct BlockMap {
 // Parts dealt from one XCD later every round instead of a part to an XCD (us, call
 // time, full windows of cached keys): 2048 queries, 15/5 heads of 64, window 8192
 // 111 -> 92; 4096, 4/2 heads, 80 -> 60.
-TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool packed) {
+//
+// Runs where the items leave a CU one workgroup more than it has to have, or an
+// XCD 3 % more than its share (us, items / runs): 1900 queries on 2047 cached keys,
+// 15/5 heads of 64, window 2048 (240 workgroups, 48 of them on one XCD) 44 / 32;
+// windows 512 / 256, 15/5 heads of 64, T = 13000 64 / 59, 2 x 18432 155 / 148. 4/2
+// heads, T = 33000, windows 1024 / 512, has 2 % more and stays with items (53; with
+// equal counts 61: its extra workgroups are the short first ones).
+TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool packed,
+                                bool even) {
   BlockMap m;
   m.nqb = nqb;
   m.npair = make_fast_div(npair);
   m.ngrp = make_fast_div(ngrp);
-  const bool queued = (int64_t)npair * nqb * ngrp > kXcd * kXcdCus;
+  const int64_t nwg = (int64_t)npair * nqb * ngrp, cus = kXcd * kXcdCus;
+  const bool queued = nwg > cus;
   int seg = 32;
   auto few = [&](int items) { return (int64_t)npair * ((nqb + seg - 1) / seg) < items; };
   while (seg > 1 && few(queued && seg > 4 ? 8 * kXcd : kXcd)) seg /= 2;
@@ -423,7 +444,35 @@ TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool pa
   m.items = levels * npair;
   m.rounds = (m.items + kXcd - 1) / kXcd;
   m.deal = npair % kXcd != 0 ? kDealSnake : alike % kXcd != 0 ? kDealTurn : kDealForth;
+  // the workgroups of the fullest XCD, by items and by runs
+  int dealt = 0;
+  const int run = (int)((nwg + kXcd - 1) / kXcd);
+  if (even ? nwg <= 32 * cus : !queued) {
+    int count[kXcd] = {};
+    for (int i = 0; i < m.items; ++i) {
+      const int round = i / kXcd, left = nqb - i / npair * m.seg;
+      const int x = ((i ^ (-(m.deal & round & 1) & (kXcd - 1))) - (round & m.deal >> 1)) & (kXcd - 1);
+      count[x] += (left < m.seg ? left : m.seg) * ngrp;
+      dealt = count[x] > dealt ? count[x] : dealt;
+    }
+  }
+  auto cu = [](int n) { return (n + kXcdCus - 1) / kXcdCus; };
+  if (cu(dealt) > cu(run) || dealt > run + run / 32) {
+    m.deal = kDealRuns;
+    m.per = make_fast_div(nqb);
+    m.seg = (int)(nwg / kXcd);
+    m.items = (int)(nwg % kXcd);
+    m.rounds = m.seg + (m.items > 0);
+  }
   return m;
+}
+
+// Whether the rows q_off .. T - 1 have (nearly) their whole window of hi keys, so
+// that every block sweeps about as many tiles: 5 % of the keys are missing at most.
+TTCD_HD bool even_rows(int T, int q_off, int hi) {
+  const int64_t first = q_off + 1, last = hi - 1;  // histories shorter than hi
+  return first > last ||
+         (last - first + 1) * (2 * (int64_t)hi - first - last) * 10 <= (int64_t)(T - q_off) * hi;
 }
 
 // Query rows per wavefront for a GQA group size (see Geometry): 16 rows of
