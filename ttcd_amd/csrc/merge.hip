@@ -95,7 +95,8 @@ hipError_t launch_typed(const MergeArgs& a, hipStream_t stream) {
 // One thread: 8 elements of one row. The parts' LSEs of a row are shared by its
 // D / 8 threads (one cache line); their outputs are read once, 32 bytes a
 // thread and part.
-template <typename T>
+// NEAR: a dual call, whose near parts also make the student's output.
+template <typename T, bool NEAR>
 __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs a) {
   const int ng = a.D / 8;
   const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -116,12 +117,22 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs a) {
     for (int p = p0; p < p1; ++p) m = fmaxf(m, a.part_lse[p * rows + li]);
     return m;
   };
-  const bool near = a.o_near != nullptr;
-  float m = largest(0, near ? a.near_parts : a.parts);
-  float ref = m == -INFINITY ? 0.f : m;  // no key in any of them: every weight is 0
-  float acc[8], sum = 0.f;
+  float acc[8], sum = 0.f, ref = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+  auto fold = [&](int p0, int p1) {
+    for (int p = p0; p < p1; ++p) {
+      const float w = expf(a.part_lse[p * rows + li] - ref);
+      const f32x4* v = reinterpret_cast<const f32x4*>(src + p * rows * a.D);
+      const f32x4 lo = __builtin_nontemporal_load(v), hi = __builtin_nontemporal_load(v + 1);
+      sum += w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        acc[e] = fmaf(lo[e], w, acc[e]);
+        acc[4 + e] = fmaf(hi[e], w, acc[4 + e]);
+      }
+    }
+  };
   auto emit = [&](void* o, float* lse) {
     const float inv = sum > 0.f ? 1.0f / sum : 0.f;
     P8<T> out;
@@ -130,29 +141,22 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs a) {
     *reinterpret_cast<u32x4*>(static_cast<T*>(o) + off) = out.raw;
     if (lse != nullptr && dg == 0) lse[li] = sum > 0.f ? ref + logf(sum) : -INFINITY;
   };
-  for (int p = 0; p < a.parts; ++p) {
-    if (p == a.near_parts && near) {
-      emit(a.o_near, a.lse_near);
-      const float far = largest(p, a.parts);
-      if (far > m) {  // the factor is 0 when no near part had a key (m = -inf)
-        const float scale = expf(m - far);
-        sum *= scale;
+  const int first = NEAR ? a.near_parts : a.parts;
+  const float far = NEAR ? largest(first, a.parts) : -INFINITY;
+  float m = largest(0, first);
+  ref = m == -INFINITY ? 0.f : m;  // no key in any of them: every weight is 0
+  fold(0, first);
+  if constexpr (NEAR) {
+    emit(a.o_near, a.lse_near);
+    if (far > m) {  // the factor is 0 when no near part had a key (m = -inf)
+      const float scale = expf(m - far);
+      sum *= scale;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc[e] *= scale;
-        m = ref = far;
-      }
+      for (int e = 0; e < 8; ++e) acc[e] *= scale;
+      ref = far;
     }
-    const float w = expf(a.part_lse[p * rows + li] - ref);
-    const f32x4* v = reinterpret_cast<const f32x4*>(src + p * rows * a.D);
-    const f32x4 lo = __builtin_nontemporal_load(v), hi = __builtin_nontemporal_load(v + 1);
-    sum += w;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      acc[e] = fmaf(lo[e], w, acc[e]);
-      acc[4 + e] = fmaf(hi[e], w, acc[4 + e]);
-    }
+    fold(first, a.parts);
   }
-  if (a.near_parts == a.parts && near) emit(a.o_near, a.lse_near);
   emit(a.o, a.lse);
 }
 
@@ -160,7 +164,11 @@ template <typename T>
 hipError_t launch_combine(const CombineArgs& a, hipStream_t stream) {
   const int64_t total = (int64_t)a.B * a.T * a.H * (a.D / 8);
   const int64_t blocks = (total + 255) / 256;
-  hipLaunchKernelGGL((attn_combine_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, stream, a);
+  const dim3 grid((unsigned)blocks);
+  if (a.o_near != nullptr)
+    hipLaunchKernelGGL((attn_combine_kernel<T, true>), grid, dim3(256), 0, stream, a);
+  else
+    hipLaunchKernelGGL((attn_combine_kernel<T, false>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
