@@ -275,8 +275,8 @@ def scan_steps(dw: torch.Tensor | None, w_cur: torch.Tensor, lr: float, nsteps: 
 
 def _scan_kernel(pd, beta, z4, zh4, W_base, out, *, lr, update_every):
     """The group loop of scanfuse.py:121-172 on the update kernels and
-    batched GEMMs. pd (B*(nchunk-1)*C, H); z4 / zh4 (B, nchunk, C, I);
-    out (B, nchunk, C, H)."""
+    batched GEMMs. pd (B*(nchunk-1)*C, H); z4 (B, nchunk, C, I), zh4 the same
+    without the last chunk; out (B, nchunk, C, H)."""
     B, nchunk, C, I = z4.shape
     K = nchunk - 1
     pdt = proj_beta_t(pd, beta, B, K, C)               # (B*K, H, C)
