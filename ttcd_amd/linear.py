@@ -23,9 +23,11 @@ MAX_COLS = 16384
 
 def _rows_for_kernel(x: torch.Tensor, w: torch.Tensor) -> int:
     """The rows of x when the kernel takes x @ w.T, else 0."""
-    if (type(x) is not torch.Tensor or type(w) not in (torch.Tensor, torch.nn.Parameter)
+    if type(x) is not torch.Tensor or x.dim() < 1 or x.numel() > MAX_ROWS * x.shape[-1]:
+        return 0  # a long call pays for no more than this
+    if (type(w) not in (torch.Tensor, torch.nn.Parameter)
             or not x.is_cuda or x.device != w.device or x.dtype not in _DT or w.dtype != x.dtype
-            or w.dim() != 2 or x.dim() < 1 or x.shape[-1] != w.shape[1] or w.shape[1] % 32
+            or w.dim() != 2 or x.shape[-1] != w.shape[1] or w.shape[1] % 32
             or w.shape[0] > MAX_COLS or w.shape[0] < 1
             or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
             or fwAD._current_level >= 0  # tangents are torch's to carry
@@ -34,8 +36,7 @@ def _rows_for_kernel(x: torch.Tensor, w: torch.Tensor) -> int:
             or not x.is_contiguous() or not w.is_contiguous()
             or x.data_ptr() % 16 or w.data_ptr() % 16):
         return 0
-    rows = x.numel() // w.shape[1] if w.shape[1] else 0
-    return rows if rows <= MAX_ROWS else 0
+    return x.numel() // w.shape[1] if w.shape[1] else 0
 
 
 def _run(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int, glu: int) -> torch.Tensor:
