@@ -404,12 +404,11 @@ struct BlockMap {
 // Blocks per item. A fixed-length call whose heads (alike of them in a row sweep
 // alike: all, the ones of a sequence, or of a part) are a multiple of the XCDs
 // gives each XCD whole heads. Otherwise: when every workgroup starts at once
-// on a CU of its own, as few items as give every XCD one (the sweep of the
-// heaviest workgroup is then the call, and it is fastest when the workgroups
-// beside it fetch the same tiles); when they queue, 8 items per XCD of at
-// least 4 blocks (whose workgroups share nearly all of their tiles) and at most
-// 32 (about what an XCD runs at once). even: all blocks sweep about as many
-// tiles.
+// on a CU of its own, a run per XCD (the sweep of the heaviest workgroup is
+// then the call, and it is fastest when the workgroups beside it fetch the same
+// tiles); when they queue, 8 items per XCD of at least 4 blocks (whose
+// workgroups share nearly all of their tiles) and at most 32 (about what an XCD
+// runs at once). even: all blocks sweep about as many tiles.
 //
 // Measured against one contiguous run per XCD (us, kernel time): packed
 // 12345 tokens in 9 sequences, 15/5 heads of 64, 153 -> 88; causal T = 8192,
@@ -420,12 +419,14 @@ struct BlockMap {
 // time, full windows of cached keys): 2048 queries, 15/5 heads of 64, window 8192
 // 111 -> 92; 4096, 4/2 heads, 80 -> 60.
 //
-// Runs where the items leave a CU one workgroup more than it has to have, or an
-// XCD 3 % more than its share (us, items / runs): 1900 queries on 2047 cached keys,
+// Runs also where the items leave a CU one workgroup more than it has to have, or
+// an XCD 3 % more than its share (us, items / runs): 1900 queries on 2047 cached keys,
 // 15/5 heads of 64, window 2048 (240 workgroups, 48 of them on one XCD) 44 / 32;
-// windows 512 / 256, 15/5 heads of 64, T = 13000 64 / 59, 2 x 18432 155 / 148. 4/2
-// heads, T = 33000, windows 1024 / 512, has 2 % more and stays with items (53; with
-// equal counts 61: its extra workgroups are the short first ones).
+// causal, 4/4 heads of 128, T = 8192 (256 workgroups, the heavy ones on 4 XCDs
+// beside each other) 134 / 129; windows 512 / 256, 15/5 heads of 64, T = 13000
+// 64 / 59, 2 x 18432 155 / 148. 4/2 heads, T = 33000, windows 1024 / 512, has 2 %
+// more and stays with items (53; with equal counts 61: its extra workgroups are
+// the short first ones).
 TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool packed,
                                 bool even) {
   BlockMap m;
@@ -436,8 +437,9 @@ TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool pa
   const bool queued = nwg > cus;
   int seg = 32;
   auto few = [&](int items) { return (int64_t)npair * ((nqb + seg - 1) / seg) < items; };
-  while (seg > 1 && few(queued && seg > 4 ? 8 * kXcd : kXcd)) seg /= 2;
-  if (!packed && alike % kXcd == 0) seg = nqb;
+  while (seg > 1 && few(seg > 4 ? 8 * kXcd : kXcd)) seg /= 2;
+  const bool whole = !packed && alike % kXcd == 0;
+  if (whole) seg = nqb;
   const int levels = (nqb + seg - 1) / seg;
   m.seg = (nqb + levels - 1) / levels;
   m.per = make_fast_div(m.seg * ngrp);
@@ -447,7 +449,7 @@ TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool pa
   // the workgroups of the fullest XCD, by items and by runs
   int dealt = 0;
   const int run = (int)((nwg + kXcd - 1) / kXcd);
-  if (even ? nwg <= 32 * cus : !queued) {
+  if (even && nwg <= 32 * cus) {
     int count[kXcd] = {};
     for (int i = 0; i < m.items; ++i) {
       const int round = i / kXcd, left = nqb - i / npair * m.seg;
@@ -457,7 +459,7 @@ TTCD_HD BlockMap make_block_map(int npair, int alike, int nqb, int ngrp, bool pa
     }
   }
   auto cu = [](int n) { return (n + kXcdCus - 1) / kXcdCus; };
-  if (cu(dealt) > cu(run) || dealt > run + run / 32) {
+  if ((!queued && !whole) || cu(dealt) > cu(run) || dealt > run + run / 32) {
     m.deal = kDealRuns;
     m.per = make_fast_div(nqb);
     m.seg = (int)(nwg / kXcd);
