@@ -17,26 +17,31 @@ from . import _lib
 
 _DT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_F16}
 
+_WEIGHTS = (torch.Tensor, torch.nn.Parameter)
+
 MAX_ROWS = 512
 MAX_COLS = 16384
 
 
 def _rows_for_kernel(x: torch.Tensor, w: torch.Tensor) -> int:
     """The rows of x when the kernel takes x @ w.T, else 0."""
-    if type(x) is not torch.Tensor or x.dim() < 1 or x.numel() > MAX_ROWS * x.shape[-1]:
+    if type(x) is not torch.Tensor or type(w) not in _WEIGHTS:
+        return 0
+    xs, ws, n = x.shape, w.shape, x.numel()
+    if len(ws) != 2 or not xs or n > MAX_ROWS * ws[1]:
         return 0  # a long call pays for no more than this
-    if (type(w) not in (torch.Tensor, torch.nn.Parameter)
-            or not x.is_cuda or x.device != w.device or x.dtype not in _DT or w.dtype != x.dtype
-            or w.dim() != 2 or x.shape[-1] != w.shape[1] or w.shape[1] % 32
-            or w.shape[0] > MAX_COLS or w.shape[0] < 1
+    N, K = ws
+    dtype = x.dtype
+    if (xs[-1] != K or K % 32 or K < 1 or N > MAX_COLS or N < 1
+            or dtype not in _DT or w.dtype != dtype or not x.is_cuda or x.device != w.device
             or (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad))
             or fwAD._current_level >= 0  # tangents are torch's to carry
             # and so are autocast's casts
-            or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype)
+            or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != dtype)
             or not x.is_contiguous() or not w.is_contiguous()
             or x.data_ptr() % 16 or w.data_ptr() % 16):
         return 0
-    return x.numel() // w.shape[1] if w.shape[1] else 0
+    return n // K
 
 
 def _run(x: torch.Tensor, w: torch.Tensor, rows: int, cols: int, glu: int) -> torch.Tensor:
