@@ -318,7 +318,7 @@ hipError_t launch_vec(const void* x, const void* w, void* y, int64_t N, int C, i
 // 7.6, 2048 x 1024 K = 5 11.3 / 6.1, 4096 x 2048 K = 9 59 / 16; rows off
 // alignment 512 x 255 3.5 / 8.3, 2048 x 2047 K = 5 20 / 9.3; f32 1024 x 512
 // K = 5 4.6 / 4.8. Large, before there was a vector form: 20480 x 1537 K = 5
-// 205 -> 30, 32768 x 2560 K = 9 835 -> 144.
+// 205 -> 30, 32768 x 2560 K = 9 835 -> 140.
 constexpr int64_t kScalarOutputs = int64_t(1) << 19;
 
 template <typename X, typename W>
