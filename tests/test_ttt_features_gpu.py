@@ -210,13 +210,16 @@ def test_empty_batches(gpu, L):
 
 @torch.inference_mode()
 def test_swiglu_output_must_hold_the_result(gpu):
-    """An output of fewer elements, another dtype or device is refused before the
-    launch; one of another shape with the same rows is not."""
+    """An output of fewer rows, another dtype or device is refused before the launch;
+    one of another shape or of more rows, whose first are written, is not."""
     g = torch.zeros(4, 32, dtype=torch.bfloat16, device=gpu)
     for out in (g.half(), g[:2], g[:, :16], g.cpu()):
         with pytest.raises(ValueError):
             ttt.swiglu(g, g, out=out)
     assert ttt.swiglu(g, g, out=g.view(2, 2, 32)).shape == (2, 2, 32)
+    x = torch.randn(4, 32, generator=torch.Generator().manual_seed(0)).to(torch.bfloat16).to(gpu)
+    more = torch.full((6, 32), 3.0, dtype=torch.bfloat16, device=gpu)
+    assert torch.equal(ttt.swiglu(x, x, out=more)[:4], ttt.swiglu(x, x)) and (more[4:] == 3.0).all()
 
 
 @pytest.mark.parametrize("L", [8, 16, 32, 40])

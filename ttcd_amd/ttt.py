@@ -66,7 +66,7 @@ def swiglu(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = None
     g_st, u_st = _row_stride(gate, "swiglu", "gate"), _row_stride(up, "swiglu", "up")
     if out is None:
         out = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
-    elif (out.shape[-1:] != gate.shape[-1:] or out.numel() != gate.numel()
+    elif (out.shape[-1:] != gate.shape[-1:] or out.numel() < gate.numel()
           or out.dtype != gate.dtype or out.device != gate.device):
         raise ValueError(f"swiglu: out must hold {tuple(gate.shape)} {gate.dtype} on "
                          f"{gate.device}, got {tuple(out.shape)} {out.dtype} on {out.device}")
