@@ -82,6 +82,10 @@ def _close(got, want, bound, dtype, what):
     (1, 70, 5000, 4, 2, 64, 4999, 4998, torch.float16),       # far part of one key
     (3, 7, 16390, 8, 2, 128, 16384, 8192, torch.bfloat16),
     (1, 200, 5100, 8, 1, 64, 6000, 5100, torch.bfloat16),     # windows past the keys: no far part
+    # 24 pairs of part and head, dealt to the XCDs from one later every round, and with
+    # whole windows in runs
+    (1, 1454, 5526, 4, 4, 64, -1, 1000, torch.bfloat16),
+    (1, 2599, 8674, 4, 4, 128, 6000, 3000, torch.float16),
 ])
 @torch.inference_mode()
 def test_split_calls_match_the_whole_call(gpu, B, Tq, Tk, H, HK, D, wt, ws, dtype):
