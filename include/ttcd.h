@@ -497,9 +497,9 @@ ttcd_status ttcd_attn_schedule_coverage(int T, int dual, int window_s,
  * no GPU needed): counts[(pair * nqb + block) * ngrp + group] += 1 for every
  * workgroup id of a launch over npair K/V heads of nqb query blocks of ngrp
  * workgroups, xcd_work[x] += its relative sweep for the ids of XCD x. packed:
- * 0 a causal call (block + 1); 1 packed sequences and 3 the parts of a split
- * call, of unequal lengths ((pair + 1) * (block + 1)); 2 rows that all have their
- * whole window (1). */
+ * 0 a causal call and 1 packed sequences (block + 1); 2 rows that all have their
+ * whole window (1); 3 the parts of a split call, of unequal lengths ((pair + 1) *
+ * (block + 1)). */
 ttcd_status ttcd_attn_block_coverage(int npair, int nqb, int ngrp, int packed,
                                      int32_t* counts, int64_t xcd_work[8]);
 

@@ -1251,7 +1251,7 @@ ttcd_status ttcd_attn_block_coverage(int npair, int nqb, int ngrp, int packed, i
     if (pair < 0 || pair >= npair || qb < 0 || qb >= nqb || grp < 0 || grp >= ngrp)
       return fail(TTCD_ERR_UNSUPPORTED, "block map error: id %d -> (%d, %d, %d)", g, pair, qb, grp);
     counts[((int64_t)pair * nqb + qb) * ngrp + grp] += 1;
-    xcd_work[g % ttcd::kXcd] += packed == 2 ? 1 : (int64_t)(qb + 1) * (packed & 1 ? pair + 1 : 1);
+    xcd_work[g % ttcd::kXcd] += packed == 2 ? 1 : (int64_t)(qb + 1) * (packed == 3 ? pair + 1 : 1);
   }
   return ok();
 }
